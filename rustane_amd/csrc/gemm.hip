@@ -110,17 +110,16 @@ int gemm_splits(int N, int T, int K, int wgs) {
 }
 
 // The residual + RMSNorm projections (gemm_residual_norm): a long reduction
-// (K >= 2N) whose 256x128 tiles in S splits fill the wgs workgroups exactly
+// (K >= 2N) whose 128x256 tiles in S splits fill the wgs workgroups exactly
 // runs on those tiles (7B W2 at 512 tokens: 64 tiles x 4 splits instead of
-// 128 of 128x128 x 2; batch-1 forward 9.40-9.44 -> 9.34-9.36 ms: the wider
-// tile reads each activation panel half as often per flop, which outweighs
-// the reduce reading 4 partials instead of 2; Wo, K = N, gains less).
+// 128 of 128x128 x 2; GEMM alone 54 -> 45.5 us: the wider tile's main loop
+// outweighs the reduce reading 4 partials instead of 2; Wo, K = N, gains less).
 // Otherwise gemm_splits on 128x128 tiles. *wide tells which.
 int gemm_norm_splits(int N, int T, int K, int wgs, bool* wide) {
   *wide = false;
   const int S = gemm_splits(N, T, K, wgs);
   if (S <= 1 || K < 2 * N) return S;
-  const long t = ntiles(N, T, 256, 128);
+  const long t = ntiles(N, T, 128, 256);
   if (t <= 0 || wgs % t) return S;
   const int Sw = (int)(wgs / t);
   if (Sw < 2 || Sw > GEMM_MAX_SPLITS || Sw * 8 > K / 64) return S;
@@ -133,7 +132,7 @@ hipError_t gemm_store(const f16* W, const f16* X, int N, int T, int K, float* C,
 }
 hipError_t gemm_residual(const f16* W, const f16* X, int N, int T, int K, const EpiResidual& e,
                          const GemmScratch* scr, hipStream_t st, int kw) {
-  return launch_gemm(W, X, N, T, K, e, scr, st, {}, kw);
+  return launch_gemm(W, X, N, T, K, e, scr, st, kw);
 }
 hipError_t gemm_residual_norm(const f16* W, const f16* X, int N, int T, int K, const EpiResidual& e,
                               const NormOut& no, const GemmScratch* scr, hipStream_t st, int kw,
@@ -146,8 +145,8 @@ hipError_t gemm_residual_norm(const f16* W, const f16* X, int N, int T, int K, c
     const size_t stride = (size_t)T * N;
     if (!scr->p || (size_t)S * stride > scr->floats || (long)N * K >= (1L << 31)) return hipErrorInvalidValue;
     const hipError_t err =
-        wide ? launch_tile<256, 128, 2, 2>(W, X, N, T, K, EpiSplit{scr->p, N, stride}, st, S, {}, kw)
-             : launch_tile<128, 128, 2, 2>(W, X, N, T, K, EpiSplit{scr->p, N, stride}, st, S, {}, kw);
+        wide ? launch_tile<128, 256>(W, X, N, T, K, EpiSplit{scr->p, N, stride}, st, S, kw)
+             : launch_tile<128, 128>(W, X, N, T, K, EpiSplit{scr->p, N, stride}, st, S, kw);
     if (err != hipSuccess) return err;
     if (mid && (err2 = hipEventRecord(mid, st)) != hipSuccess) return err2;
     // 1..8: whole multiples of 1024; 9..16: ragged, ceil(N / 1024) = 1..8
@@ -168,7 +167,7 @@ hipError_t gemm_residual_norm(const f16* W, const f16* X, int N, int T, int K, c
     }
     return hipGetLastError();
   }
-  const hipError_t err = launch_gemm(W, X, N, T, K, e, nullptr, st, {}, kw);
+  const hipError_t err = launch_gemm(W, X, N, T, K, e, nullptr, st, kw);
   if (err != hipSuccess) return err;
   if (mid && (err2 = hipEventRecord(mid, st)) != hipSuccess) return err2;
   return rmsnorm(e.out, N, no.gamma, T, N, no.eps, no.xn, nullptr, st, no.split);

@@ -1,12 +1,22 @@
-// Prefill GEMM kernel (launch policy in gemm_launch.hpp).
+// Prefill GEMM kernels (launch policy in gemm_launch.hpp): gemm_nt_kernel for
+// tiles of at least 192x128 or 128x256, gemm_nt_kernel_reg for smaller ones.
 //
-// C^T tile = W_tile · X_tile^T on v_mfma_f32_32x32x16_f16:
+// C^T tile = W_tile · X_tile^T on v_mfma_f32_{16x16x32,32x32x16}_f16:
 //   W [N, K] fp16, K contiguous (weights repacked output-major at upload)
 //   X [T, K] fp16, K contiguous (token-major activations)
 //   result(t, f) = sum_k X[t,k] * W[f,k], fp32 accumulate, handed to an epilogue.
 // MFMA rows are output features and MFMA columns are tokens, so each lane ends
 // up holding 4 consecutive features of one token — the shape every epilogue
-// (RoPE pairs, SwiGLU pairs, residual float4) wants.
+// (RoPE pairs, SwiGLU pairs, residual float4) wants. The two instruction
+// shapes give the same bits.
+//
+// Split-K: blockIdx.y selects one of gridDim.y contiguous ranges of 64-wide K
+// slices (kq slices each, the last one shorter); with gridDim.y = 1 the range
+// is all of K. Each split hands its partial sums to the epilogue (EpiSplit).
+//
+// Split X rows (common.hpp): X rows hold K = 2*kw halves [hi | lo] while W
+// rows hold kw; k-slice k0 reads W columns k0 mod kw, so the hi and the lo
+// halves of each row meet the same weights. kw = K otherwise.
 //
 // LDS rows are 128 B (64 halfs) of eight 16-byte chunks; chunk c of row r is
 // stored at c ^ swz(r), which keeps both the loaders' ds_write_b128 and the
@@ -79,6 +89,349 @@ struct EpiSumSq : std::false_type {};
 template <class E>
 struct EpiSumSq<E, std::void_t<decltype(E::kSumSq)>> : std::bool_constant<E::kSumSq> {};
 
+// Tile order: groups of GM weight-row panels, token tiles iterated inside a
+// group (tile = group*GM*ntt + tt*rows + row), and each XCD takes a
+// contiguous range of that order. With 8+ token tiles the 32 tiles an XCD
+// runs at a time then share 8 weight panels and 4 token panels in its L2
+// instead of 2 and 16 (7B at 4096 tokens: W1|W3 749 -> 663 us, QKV 372 ->
+// 338 us); with fewer token tiles GM = 1 (plain row-major order) measures
+// ~1% better.
+HB_DEV void tile_of(int nft, int ntt, int& tile, int& ft, int& tt) {
+  const int GM = ntt >= 8 ? 8 : 1;
+  tile = xcd_remap(blockIdx.x, nft * ntt);
+  const int grp = tile / (GM * ntt), rem = tile - grp * (GM * ntt);
+  const int rows = min(GM, nft - grp * GM);
+  tt = rem / rows;
+  ft = grp * GM + (rem - tt * rows);
+}
+
+// Issue schedule of gemm_nt_kernel's LDS copies, as seen by one wave: per K
+// slice of 64 each wave issues one 1 KB copy per 32-row weight block of the
+// wave grid (W_i, i < FM) and two per 128-token block (X_j, j < TM), in the
+// order below; cum(p) counts those issued by the end of phase p, wait(p) is
+// the largest number of copies that may still be in flight at the end of
+// phase p's memory half so that everything phase p + 1 reads has landed.
+//   phase 0: W_{FM-1} of slice k+1, X_0 of slice k+2
+//   phase 1: X_1 of slice k+2        (FM == 2: also W_0 of k+2)
+//   phase 2: W_0, W_1 of slice k+2
+//   phase 3: W_2 of slice k+2
+// W_i is read from LDS in phase i, X_j in phase FM - TM + j of the slice
+// before, each at least one phase before its buffer is copied into again.
+template <int FT, int TT>
+struct GemmPlan {
+  static constexpr int FM = FT / 64, TM = TT / 128, N = FM + 2 * TM;
+  static_assert(FT % 64 == 0 && TT % 128 == 0 && FM >= 2 && FM <= 4 && TM >= 1 && TM <= 2, "tile");
+  static constexpr int cum(int p) {
+    int c = 3;
+    if (FM == 2) return p >= 1 ? N : c;
+    if (p >= 1) c += 2 * (TM - 1);
+    if (p >= 2) c += 2;
+    if (p >= 3) c += 1;
+    return c;
+  }
+  static constexpr int wait(int p) {
+    const int k = 4, issued = k * N + cum(p);  // any slice k: the differences do not depend on it
+    const int kr = p + 1 == FM ? k + 1 : k, ph = p + 1 == FM ? 0 : p + 1;  // slice and phase that read
+    // index of W_ph(kr)'s copy in issue order
+    int first = ph == FM - 1 ? (kr - 1) * N : (kr - 2) * N + 1 + 2 * TM + ph;
+    int w = issued - 1 - first;
+    for (int j = 0; j < TM; ++j)
+      if (ph == FM - TM + j) {  // X_j(kr + 1), second copy
+        const int v = issued - 1 - ((kr - 1) * N + 2 + 2 * j);
+        if (v < w) w = v;
+      }
+    return w;
+  }
+};
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+// One wave copies 64 x 16 bytes from global memory (per-lane byte offset voff,
+// wave-uniform soff) straight into LDS at lds + 16 * lane. No output register;
+// the copy is counted by vmcnt (dma_wait). The nop is the wait state between
+// the write of m0 and its use.
+HB_DEV void dma_1k(uint32_t lds, uint32_t voff, i32x4 rsrc, uint32_t soff) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc),
+      "s"(soff)
+      : "memory");
+}
+// At most N of this wave's copies in flight; all its LDS reads done.
+template <int N>
+HB_DEV void dma_wait() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+// Barrier without the vmcnt drain of __syncthreads.
+HB_DEV void raw_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The GEMM kernel: 8 waves (2 feature rows x 4 token columns), two per SIMD,
+// on v_mfma_f32_16x16x32_f16.
+//
+// Operand tiles go from global memory straight into LDS (buffer_load ... lds,
+// no registers), two 64-wide K slices deep; wave (wf, wt) owns the features
+// i*64 + wf*32 .. +32 (i < FM) and the tokens j*128 + wt*32 .. +32 (j < TM). A
+// slice is FM phases; phase i reads the 32-feature fragments of block i
+// (and, in the last TM phases, the next slice's token fragments), issues the
+// copies of GemmPlan and then runs the 8 * TM MFMAs of its accumulator row.
+// Each phase has two halves separated by barriers -- LDS reads and copies,
+// then MFMAs -- and the waves of the second feature row run half a phase
+// behind those of the first, so on every SIMD one wave feeds the matrix core
+// while the other reads and issues (s_setprio favours the one in its MFMA
+// half). Each LDS region (one W_i or X_j) is refilled as soon as both halves
+// have read it, about 1.5 slices before its next use, and the waits count
+// copies (dma_wait) instead of draining them.
+//
+// What bounds it: the chip's power limit. MFMA busy is ~83% of the active
+// cycles (63% in the 4-wave register-staged kernel below at 4096 tokens), and
+// the clock then settles with the energy per flop, so the instruction shape
+// matters: 16x16x32 touches half the accumulator registers per flop of
+// 32x32x16 and took the same schedule from 393 to 328 us on 12288 x 4096 x
+// 4096 (results bit-identical), and consecutive MFMAs that keep the token
+// operand another 2-4%. Before -> after, fp32 output, back to back on one
+// box (N x T x K): 12288 x 4096 x 4096 413 -> 307 us (998 -> 1344 TFLOP/s),
+// 22016 x 4096 x 4096 691 -> 608 us, 4096 x 4096 x 11008 287 -> 256 us,
+// 8192^3 886 -> 751 us (1463 TFLOP/s), 22016 x 512 x 4096 87 -> 76 us.
+//
+// LDS is written by copies the compiler does not see: its address enters
+// their asm, and every copy is waited for before the barrier that precedes its
+// reads. Past the last slice the copies re-read the last slice, so every
+// phase has the same shape; they are drained before LDS is used again.
+template <int FT, int TT, class Epi>
+__global__ __launch_bounds__(512, 1) void gemm_nt_kernel(const f16* __restrict__ W, const f16* __restrict__ X,
+                                                         int N, int T, int K, int kw, int kq, Epi epi) {
+  using P = GemmPlan<FT, TT>;
+  constexpr int NT = 512, FM = P::FM, TM = P::TM;
+  constexpr uint32_t STAGE = (FT + TT) * 128, XOFF = FT * 128;  // bytes
+  __shared__ f16x8 smem[2 * (FT + TT) * 8];  // [stage][W rows, X rows][8 swizzled chunks]
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
+  const int wf = wave >> 2, wt = wave & 3;
+  int tile, ft, tt;
+  tile_of((N + FT - 1) / FT, (T + TT - 1) / TT, tile, ft, tt);
+  const int f_base = ft * FT, t_base = tt * TT;
+
+  // Copies: one instruction fills 8 rows of 128 bytes; lane l writes chunk l%8
+  // of row l/8, so it reads source chunk (l%8) ^ swz(row). Instruction n of
+  // wave w takes rows n*64 + w*8 .. +8 of its operand. Byte offsets are
+  // 32-bit: the launchers keep N*K and T*K below 2^31 elements.
+  const int lr = lane >> 3, lc = (lane & 7) ^ lr ^ (wave & 1);
+  uint32_t wvo[FM], xvo[2 * TM];
+#pragma unroll
+  for (int i = 0; i < FM; ++i) wvo[i] = (uint32_t)(min(f_base + i * 64 + wave * 8 + lr, N - 1) * kw + lc * 8) * 2u;
+#pragma unroll
+  for (int j = 0; j < 2 * TM; ++j) xvo[j] = (uint32_t)(min(t_base + j * 64 + wave * 8 + lr, T - 1) * K + lc * 8) * 2u;
+  const uint64_t wa = (uint64_t)W, xa = (uint64_t)X;
+  const i32x4 wrs = {(int)(uint32_t)wa, (int)(uint32_t)(wa >> 32), -1, 0x00020000};
+  const i32x4 xrs = {(int)(uint32_t)xa, (int)(uint32_t)(xa >> 32), -1, 0x00020000};
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) f16x8*)smem + wave * 1024;
+  const int kt0 = blockIdx.y * kq;
+  const int nk = min(kq, K / 64 - kt0);
+  auto dma_w = [&](int i, int stage, int k) {
+    const int k0 = (kt0 + min(k, nk - 1)) * 64;
+    dma_1k(lds0 + stage * STAGE + i * 8192, wvo[i], wrs, (uint32_t)(k0 < kw ? k0 : k0 - kw) * 2u);
+  };
+  auto dma_x = [&](int j, int stage, int k) {
+    const uint32_t so = (uint32_t)(kt0 + min(k, nk - 1)) * 128u;
+    dma_1k(lds0 + stage * STAGE + XOFF + (2 * j) * 8192, xvo[2 * j], xrs, so);
+    dma_1k(lds0 + stage * STAGE + XOFF + (2 * j + 1) * 8192, xvo[2 * j + 1], xrs, so);
+  };
+
+  // acc[i][j][g]: 16x16 block (feature half g>>1, token half g&1) of block (i, j)
+  f32x4 acc[FM][TM][4];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) acc[i][j][g] = f32x4{};
+
+  // fragment s of a 32-row block: its rows (s>>1)*16 + lane%16, k (s&1)*32 + 8*(lane/16)
+  const int l16 = lane & 15, quad = lane >> 4;
+  int ao[4], bo[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int row = (s >> 1) * 16 + l16, c = ((s & 1) * 4 + quad) ^ lds_swz(row);
+    ao[s] = (wf * 32 + row) * 8 + c;
+    bo[s] = FT * 8 + (wt * 32 + row) * 8 + c;
+  }
+  f16x8 a[4], b[2][TM][4];
+
+  // Prologue: the copies of issue slices -2 and -1, then slice 0's token fragments.
+#pragma unroll
+  for (int j = 0; j < TM; ++j) dma_x(j, 0, 0);
+#pragma unroll
+  for (int i = 0; i < FM; ++i) dma_w(i, 0, 0);
+#pragma unroll
+  for (int j = 0; j < TM; ++j) dma_x(j, 1, 1);
+#pragma unroll
+  for (int i = 0; i < FM - 1; ++i) dma_w(i, 1, 1);
+  dma_wait<P::wait(FM - 1)>();
+  raw_barrier();
+#pragma unroll
+  for (int j = 0; j < TM; ++j)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) b[0][j][s] = smem[bo[s] + j * 1024];
+  dma_wait<63>();
+  raw_barrier();
+  if (wf == 1) raw_barrier();  // the second feature row runs half a phase behind
+
+  auto slice = [&](auto sc, int k) {
+    constexpr int S = decltype(sc)::value;
+    static_for<0, FM>([&](auto pc) {
+      constexpr int p = decltype(pc)::value;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) a[s] = smem[S * (STAGE / 16) + ao[s] + p * 512];
+      if constexpr (p >= FM - TM) {
+        constexpr int j = p - (FM - TM);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) b[S ^ 1][j][s] = smem[(S ^ 1) * (STAGE / 16) + bo[s] + j * 1024];
+      }
+      if constexpr (p == 0) {
+        dma_w(FM - 1, S ^ 1, k + 1);
+        dma_x(0, S, k + 2);
+      }
+      if constexpr (p == 1 && TM == 2) dma_x(1, S, k + 2);
+      if constexpr (p == 1 && FM == 2) dma_w(0, S, k + 2);
+      if constexpr (p == 2) {
+        dma_w(0, S, k + 2);
+        dma_w(1, S, k + 2);
+      }
+      if constexpr (p == 3) dma_w(2, S, k + 2);
+      dma_wait<P::wait(p)>();
+      raw_barrier();
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+          for (int jh = 0; jh < 2; ++jh)
+#pragma unroll
+            for (int ih = 0; ih < 2; ++ih)
+              acc[p][j][ih * 2 + jh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                  a[ih * 2 + s], b[S][j][jh * 2 + s], acc[p][j][ih * 2 + jh], 0, 0, 0);
+      __builtin_amdgcn_s_setprio(0);
+      raw_barrier();
+    });
+  };
+  // nk >= 1 for every split (the launcher checks (splits - 1) * kq < K / 64)
+  int k = 0;
+  for (; k + 2 <= nk; k += 2) {
+    slice(std::integral_constant<int, 0>{}, k);
+    slice(std::integral_constant<int, 1>{}, k + 1);
+  }
+  if (k < nk) slice(std::integral_constant<int, 0>{}, k);
+  if (wf == 0) raw_barrier();
+  dma_wait<0>();
+
+  using AX = EpiAux<Epi>;
+  using AuxT = typename AX::type;
+  // a staged table of up to 32 float4 per token (hd <= 128) fits in the
+  // operand LDS, its first half in 16*FT float4 and its second in the 16*TT
+  // after them, when TT <= FT; staged on the 256-feature tiles, whose long
+  // epilogues gain (7B QKV at 4096 tokens 424 -> 392 us, 5B at 2048 tokens
+  // 105 -> 100 us), not on 128x128 (600M QKV 25.6 -> 26.6 us)
+  constexpr bool STAGED = EpiStage<Epi>::value && TT <= FT && FT == 256;
+  float4* const stab_lo = reinterpret_cast<float4*>(smem);
+  float4* const stab_hi = stab_lo + 16 * FT;
+  if constexpr (STAGED) {
+    raw_barrier();  // every wave's copies are in, every wave's reads done
+    epi.template stage<TT, NT>(stab_lo, stab_hi, t_base, f_base, tid);
+    __syncthreads();
+  }
+
+  // Epilogue over the FM x 2*TM x 2 accumulator quads as straight-line code: a
+  // loop would be left rolled once the epilogue body is large, and indexing
+  // acc with a loop counter moves the whole accumulator array to scratch
+  // memory. Operands that epilogues read from memory (residual stream, RoPE
+  // table) are loaded one accumulator row ahead of the stores: the loads
+  // cannot be moved above stores that might alias them, so a load-store-load
+  // chain per quad would expose the load latency once per quad.
+  // Quad q of row i: token half q>>1 (of 2*TM), feature half q&1.
+  AuxT aux[2][TM * 4];
+  auto tok = [&](int jt) { return t_base + (jt >> 1) * 128 + wt * 32 + (jt & 1) * 16 + l16; };
+  auto fblk = [&](int i) { return f_base + i * 64 + wf * 32; };  // wave-uniform
+  auto feat = [&](int i, int ih) { return fblk(i) + ih * 16 + quad * 4; };
+  auto load_row = [&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    static_for<0, TM * 4>([&](auto qc) {
+      constexpr int q = decltype(qc)::value;
+      const int t = tok(q >> 1), f = feat(i, q & 1);
+      if constexpr (STAGED) {
+        if (t < T && f < N) aux[i & 1][q] = epi.load_staged(stab_lo, stab_hi, t - t_base, TT, f, fblk(i));
+      } else {
+        if (t < T && f < N) aux[i & 1][q] = AX::load(epi, t, f, fblk(i));
+      }
+    });
+  };
+  load_row(std::integral_constant<int, 0>{});
+  // EpiRows: the token part of the output addresses once per token, the
+  // (feature block, token) part once per 2 quads, both outside the quads'
+  // bounds tests (they read no memory)
+  constexpr bool ROWS = EpiRows<Epi>::value;
+  static_assert(!ROWS || !EpiSumSq<Epi>::value, "row-addressed epilogues return nothing");
+  typename EpiRows<Epi>::Tok tkj[ROWS ? 2 * TM : 1];
+  if constexpr (ROWS) {
+    static_for<0, 2 * TM>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      tkj[j] = epi.tok(tok(j));
+    });
+  }
+  float lane_sq = 0.f;
+  static_for<0, FM>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    if constexpr (i + 1 < FM) load_row(std::integral_constant<int, i + 1>{});
+    static_for<0, 2 * TM>([&](auto jc) {
+      constexpr int jt = decltype(jc)::value;
+      const int t = tok(jt);
+      if constexpr (ROWS) {
+        const auto rc = epi.row(tkj[jt], fblk(i));
+        static_for<0, 2>([&](auto hc) {
+          constexpr int ih = decltype(hc)::value;
+          const int f = feat(i, ih);
+          if (t < T && f < N)
+            epi.store_row(rc, f, acc[i][jt >> 1][ih * 2 + (jt & 1)], aux[i & 1][2 * jt + ih], fblk(i));
+        });
+      } else {
+        static_for<0, 2>([&](auto hc) {
+          constexpr int ih = decltype(hc)::value;
+          const int f = feat(i, ih);
+          if (t < T && f < N) {
+            const f32x4 v = acc[i][jt >> 1][ih * 2 + (jt & 1)];
+            if constexpr (EpiSumSq<Epi>::value)
+              lane_sq += AX::apply(epi, t, f, v, aux[i & 1][2 * jt + ih], fblk(i));
+            else
+              AX::apply(epi, t, f, v, aux[i & 1][2 * jt + ih], fblk(i));
+          }
+        });
+      }
+    });
+  });
+  if constexpr (EpiSumSq<Epi>::value) {
+    float* red = (float*)smem;
+    const float s = wave_sum(lane_sq);
+    raw_barrier();  // every wave's copies are in: the operand buffers are free
+    if (lane == 0) red[wave] = s;
+    __syncthreads();
+    if (tid == 0) {
+      float tot = 0.f;
+#pragma unroll
+      for (int w = 0; w < NT / 64; ++w) tot += red[w];
+      epi.sq_out[tile] = tot;
+    }
+  }
+}
+
+// The small-tile kernel: 4 waves of 32x32x16 MFMAs with register-staged operands.
+// Its 128x128 tiles run two to a CU, where gemm_nt_kernel has too little work
+// per phase to gain (4096 x 512 x 4096 in two splits: 23.4 against 23.3 us, 600M
+// QKV 4608 x 512 x 1536 16.2 against 17.5 us).
+//
 // Pipeline: two 64-wide K slices are in flight in registers while the MFMAs
 // consume a third from LDS. Iteration k computes slice k from LDS buffer k&1,
 // issues the global loads of slice k+2 into register set k&1 and writes slice
@@ -96,25 +449,11 @@ struct EpiSumSq<E, std::void_t<decltype(E::kSumSq)>> : std::bool_constant<E::kSu
 // (one wave per SIMD has nothing else to issue).
 // Past the last slice the loads re-read the last slice (clamped), so every
 // iteration has the same shape.
-//
-// Split-K: blockIdx.y selects one of gridDim.y contiguous ranges of 64-wide K
-// slices (kq slices each, the last one shorter); with gridDim.y = 1 the range
-// is all of K. Each split hands its partial sums to the epilogue (EpiSplit).
-//
-// Batches: blockIdx.z selects one of gridDim.z independent products whose
-// operands start wbs and xbs halfs apart (attention backward: one per
-// sequence and KV head); epilogues that care read blockIdx.z themselves.
-//
-// Split X rows (common.hpp): X rows hold K = 2*kw halves [hi | lo] while W
-// rows hold kw; k-slice k0 reads W columns k0 mod kw, so the hi and the lo
-// halves of each row meet the same weights. kw = K otherwise.
 template <int FT, int TT, int WF, int WT, class Epi>
-__global__ __launch_bounds__(WF* WT * 64, 1) void gemm_nt_kernel(const f16* __restrict__ W,
+__global__ __launch_bounds__(WF* WT * 64, 1) void gemm_nt_kernel_reg(const f16* __restrict__ W,
                                                                  const f16* __restrict__ X, int N,
                                                                  int T, int K, int kw, int kq,
-                                                                 Epi epi, size_t wbs, size_t xbs) {
-  W += blockIdx.z * wbs;
-  X += blockIdx.z * xbs;
+                                                                 Epi epi) {
   constexpr int NT = WF * WT * 64;
   constexpr int WFT = FT / WF, WTT = TT / WT;
   constexpr int FM = WFT / 32, TM = WTT / 32;
@@ -132,19 +471,8 @@ __global__ __launch_bounds__(WF* WT * 64, 1) void gemm_nt_kernel(const f16* __re
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
   const int wf = wave / WT, wt = wave - wf * WT;
-  const int nft = (N + FT - 1) / FT, ntt = (T + TT - 1) / TT;
-  // Tile order: groups of GM weight-row panels, token tiles iterated inside a
-  // group (tile = group*GM*ntt + tt*rows + row), and each XCD takes a
-  // contiguous range of that order. With 8+ token tiles the 32 tiles an XCD
-  // runs at a time then share 8 weight panels and 4 token panels in its L2
-  // instead of 2 and 16 (7B at 4096 tokens: W1|W3 749 -> 663 us, QKV 372 ->
-  // 338 us); with fewer token tiles GM = 1 (plain row-major order) measures
-  // ~1% better.
-  const int GM = ntt >= 8 ? 8 : 1;
-  const int tile = xcd_remap(blockIdx.x, nft * ntt);
-  const int grp = tile / (GM * ntt), rem = tile - grp * (GM * ntt);
-  const int rows = min(GM, nft - grp * GM);
-  const int tt = rem / rows, ft = grp * GM + (rem - tt * rows);
+  int tile, ft, tt;
+  tile_of((N + FT - 1) / FT, (T + TT - 1) / TT, tile, ft, tt);
   const int f_base = ft * FT, t_base = tt * TT;
 
   const int r0 = tid >> 3, c0 = tid & 7;
@@ -258,23 +586,9 @@ __global__ __launch_bounds__(WF* WT * 64, 1) void gemm_nt_kernel(const f16* __re
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // Epilogue operands read from memory: all of them before the main loop when
-  // they fit in 96 registers and the tile runs one wave per SIMD anyway
-  // (192x128 and larger; their latency then hides behind the K loop), else one
-  // accumulator row at a time (see the epilogue).
   using AX = EpiAux<Epi>;
   using AuxT = typename AX::type;
-  constexpr bool HOIST =
-      !std::is_empty_v<AuxT> && FM * TM * 4 * sizeof(AuxT) <= 96 * 4 && FT * TT >= 192 * 128;
-  // a staged table of up to 32 float4 per token (hd <= 128) fits in the
-  // operand LDS, its first half in sW (16*FT float4) and its second in sX
-  // (16*TT), when TT <= FT; staged on the 256-feature tiles, whose long
-  // epilogues gain (7B QKV at 4096 tokens 424 -> 392 us, 5B at 2048 tokens
-  // 105 -> 100 us), not on 128x128 (600M QKV 25.6 -> 26.6 us)
-  constexpr bool STAGE = EpiStage<Epi>::value && !HOIST && TT <= FT && FT == 256;
-  float4* const stab_lo = reinterpret_cast<float4*>(&sW[0][0]);
-  float4* const stab_hi = reinterpret_cast<float4*>(&sX[0][0]);
-  AuxT aux[HOIST ? FM : 2][TM * 4];
+  AuxT aux[2][TM * 4];
   auto tok = [&](int j) { return t_base + wt * WTT + j * 32 + (lane & 31); };
   auto fblk = [&](int i) { return f_base + wf * WFT + i * 32; };  // wave-uniform
   auto feat = [&](int i, int g) { return fblk(i) + 8 * g + 4 * khalf; };
@@ -283,15 +597,9 @@ __global__ __launch_bounds__(WF* WT * 64, 1) void gemm_nt_kernel(const f16* __re
     static_for<0, TM * 4>([&](auto qc) {
       constexpr int q = decltype(qc)::value;
       const int t = tok(q / 4), f = feat(i, q % 4);
-      if constexpr (STAGE) {
-        if (t < T && f < N)
-          aux[HOIST ? i : (i & 1)][q] = epi.load_staged(stab_lo, stab_hi, t - t_base, TT, f, fblk(i));
-      } else {
-        if (t < T && f < N) aux[HOIST ? i : (i & 1)][q] = AX::load(epi, t, f, fblk(i));
-      }
+      if (t < T && f < N) aux[i & 1][q] = AX::load(epi, t, f, fblk(i));
     });
   };
-  if constexpr (HOIST) static_for<0, FM>([&](auto ic) { load_row(ic); });
 
   // nk >= 1 for every split (the launcher checks (splits - 1) * kq < K / 64)
   gload(R0{}, kslice(0));
@@ -304,20 +612,9 @@ __global__ __launch_bounds__(WF* WT * 64, 1) void gemm_nt_kernel(const f16* __re
     iter(R1{}, kt + 1);
   }
   if (kt < nk) iter(R0{}, kt);
-  if constexpr (STAGE) {  // the main loop ended on a barrier: the operand LDS is free
-    epi.template stage<TT, NT>(stab_lo, stab_hi, t_base, f_base, tid);
-    __syncthreads();
-  }
-
-  // Epilogue over the FM x TM x 4 accumulator quads as straight-line code: a
-  // loop would be left rolled once the epilogue body is large (EpiQKV on
-  // 256x256 tiles), and indexing acc with a loop counter moves the whole
-  // accumulator array to scratch memory. The operands that epilogues read from
-  // memory (residual stream, RoPE table) were loaded before the main loop
-  // (HOIST) or are loaded one accumulator row ahead of the stores: the loads
-  // cannot be moved above stores that might alias them, so a load-store-load
-  // chain per quad would expose the load latency once per quad.
-  if constexpr (!HOIST) load_row(std::integral_constant<int, 0>{});
+  // Straight-line epilogue with the operands one accumulator row ahead, as in
+  // gemm_nt_kernel.
+  load_row(std::integral_constant<int, 0>{});
   // EpiRows: the token part of the output addresses once per token, the
   // (feature block, token) part once per 4 quads, both outside the quads'
   // bounds tests (they read no memory)
@@ -333,7 +630,7 @@ __global__ __launch_bounds__(WF* WT * 64, 1) void gemm_nt_kernel(const f16* __re
   float lane_sq = 0.f;
   static_for<0, FM>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
-    if constexpr (!HOIST && i + 1 < FM) load_row(std::integral_constant<int, i + 1>{});
+    if constexpr (i + 1 < FM) load_row(std::integral_constant<int, i + 1>{});
     if constexpr (ROWS) {
       static_for<0, TM>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
@@ -347,7 +644,7 @@ __global__ __launch_bounds__(WF* WT * 64, 1) void gemm_nt_kernel(const f16* __re
             v.y = acc[i][j][4 * g + 1];
             v.z = acc[i][j][4 * g + 2];
             v.w = acc[i][j][4 * g + 3];
-            epi.store_row(rc, f, v, aux[HOIST ? i : (i & 1)][q], fblk(i));
+            epi.store_row(rc, f, v, aux[i & 1][q], fblk(i));
           }
         });
       });
@@ -363,9 +660,9 @@ __global__ __launch_bounds__(WF* WT * 64, 1) void gemm_nt_kernel(const f16* __re
           v.z = acc[i][j][4 * g + 2];
           v.w = acc[i][j][4 * g + 3];
           if constexpr (EpiSumSq<Epi>::value)
-            lane_sq += AX::apply(epi, t, f, v, aux[HOIST ? i : (i & 1)][q], fblk(i));
+            lane_sq += AX::apply(epi, t, f, v, aux[i & 1][q], fblk(i));
           else
-            AX::apply(epi, t, f, v, aux[HOIST ? i : (i & 1)][q], fblk(i));
+            AX::apply(epi, t, f, v, aux[i & 1][q], fblk(i));
         }
       });
     }

@@ -13,15 +13,10 @@ struct GemmScratch {
   int wgs = 256;  // workgroups the split count aims for (gemm_splits)
 };
 constexpr int GEMM_MAX_SPLITS = 8;
-// One product, or n of them with operands wbs / xbs halfs apart (blockIdx.z).
-struct GemmBatch {
-  int n = 1;
-  size_t wbs = 0, xbs = 0;
-};
 // Number of K splits the residual GEMM uses for this shape when given scratch
 // (1 = none), aiming at wgs workgroups; it needs splits * T * N floats.
 int gemm_splits(int N, int T, int K, int wgs = 256);
-// The same for gemm_residual_norm, which may use 256x128 tiles (*wide) for
+// The same for gemm_residual_norm, which may use 128x256 tiles (*wide) for
 // long reductions; it needs splits * T * N floats too.
 int gemm_norm_splits(int N, int T, int K, int wgs, bool* wide);
 hipError_t gemm_store(const f16* W, const f16* X, int N, int T, int K, float* C, hipStream_t st);
@@ -57,15 +52,15 @@ hipError_t gemm_qkv(const f16* W, const f16* X, int N, int T, int K, const EpiQK
 hipError_t gemm_store_split(const f16* W, const f16* X, int N, int T, int K, float* C,
                             const GemmScratch* scr, hipStream_t st, float scale = 1.0f);
 // Weight gradient g[t, f] (+)= sum_k X[t,k] W[f,k]: accumulate (EpiAccum) or,
-// when the arena is known to be zero, store. With short K (<= 1024 tokens) the
-// fp32 read-modify-write dominates: 128x128 tiles (two per CU) when there are
-// enough of them.
+// when the arena is known to be zero, store. The usual tile choice at every K:
+// at K = 512 (22016 x 4096 outputs) 256x256 tiles take 144.5 us and 128x128
+// ones, two to a CU, 168 us.
 // With sq_out, one sum of squares of the written gradient per output tile
 // goes to sq_out[0 .. *sq_tiles) (gemm_wgrad_max_tiles bounds the count).
 hipError_t gemm_wgrad(const f16* W, const f16* X, int N, int T, int K, float* g, int ld,
                       bool accumulate, hipStream_t st, float scale = 1.0f, float* sq_out = nullptr,
                       int* sq_tiles = nullptr);
-inline long gemm_wgrad_max_tiles(int N, int T) { return (long)((N + 127) / 128) * ((T + 127) / 128); }
+inline long gemm_wgrad_max_tiles(int N, int T) { return (long)((N + 63) / 64) * ((T + 127) / 128); }
 hipError_t gemm_silu_bwd(const f16* W, const f16* X, int N, int T, int K, const EpiSiluBwd& e,
                          hipStream_t st);
 hipError_t gemm_heads(const f16* W, const f16* X, int N, int T, int K, const EpiHeads& e,

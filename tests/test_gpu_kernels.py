@@ -49,6 +49,29 @@ def test_gemm_nt_matches_float64(gpu, M, N, K):
     assert err < 1e-4 * K, err
 
 
+@pytest.mark.parametrize("K", [64, 192, 320])  # 1, 3 and 5 slices: both ends of the two-slice loop
+@pytest.mark.parametrize("M,N", [
+    (4093, 4092),   # 256x256 tiles, ragged last row and column of tiles
+    (509, 22012),   # 192x256
+    (2047, 4092),   # 128x256
+    (511, 12284),   # 192x128
+    (45, 22016),    # 128x128
+])
+def test_gemm_nt_tiles_exact(gpu, M, N, K):
+    """Small integers: every product and partial sum is exact in fp32, so any
+    order of the sums gives the same bits as the reference."""
+    import torch
+    print(f"gemm tiles M={M} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    a = rng.integers(-3, 4, (M, K)).astype(np.float32)
+    b = rng.integers(-3, 4, (N, K)).astype(np.float32)
+    da, db = to_dev(a, torch.float16), to_dev(b, torch.float16)
+    dc = torch.full((M, N), float("nan"), device="cuda")
+    hb.call("hb_op_gemm_nt", gpu.handle, da.data_ptr(), db.data_ptr(), dc.data_ptr(), M, N, K)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(dc.cpu().numpy(), a @ b.T)
+
+
 def test_gemm_nt_mfma_layout_one_hot(gpu):
     """A one-hot A row selects exactly one B row: catches any lane/register
     layout mistake in the MFMA fragments independently of rounding."""
