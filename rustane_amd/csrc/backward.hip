@@ -109,35 +109,80 @@ hipError_t cast_transpose(const float* src, int R, int C, float scale, f16* rm, 
 // dl = (p - onehot(y)) * gs with gs = loss_scale / S, times (1 - tc^2) with
 // tc = z / softcap when the logits went through softcap * tanh(. / softcap).
 // Written as fp16 [T][Vp], columns [V, Vp) zero.
-__global__ __launch_bounds__(256) void ce_backward_kernel(const float* __restrict__ logits,
-                                                          const uint32_t* __restrict__ tgt, int V,
-                                                          int Vp, float gs, float softcap,
-                                                          f16* __restrict__ dl) {
-  __shared__ float red[4];
+//
+// HBM-bound: 4 V bytes read and 2 Vp written per position. The row stays in
+// registers (NV float4 per thread, V <= 2048 * NV), so it is read once with
+// 16-byte loads and each exponential is taken once: 2048 x 32000 from 230 us
+// (three passes of 4-byte loads) to CE_BWD_US. NV = 0: any V, in three passes.
+constexpr int CE_NT = 512;
+template <int NV>
+__global__ __launch_bounds__(CE_NT) void ce_backward_kernel(const float* __restrict__ logits,
+                                                            const uint32_t* __restrict__ tgt, int V,
+                                                            int Vp, float gs, float softcap,
+                                                            f16* __restrict__ dl) {
+  constexpr int NW = CE_NT / 64;
+  __shared__ float red[NW];
   const int t = blockIdx.x;
   const float* z = logits + (size_t)t * V;
-  float m = -INFINITY;
-  for (int v = threadIdx.x; v < V; v += 256) m = fmaxf(m, z[v]);
-  m = block_max<4>(m, red);
-  float se = 0.f;
-  for (int v = threadIdx.x; v < V; v += 256) se += expf(z[v] - m);
-  se = block_sum<4>(se, red);
-  const float inv = 1.0f / se;
   const uint32_t y = tgt[t];
   const float ic = softcap > 0.f ? 1.0f / softcap : 0.f;
   f16* o = dl + (size_t)t * Vp;
-  for (int v = threadIdx.x; v < Vp; v += 256) {
-    float d = 0.f;
-    if (v < V) {
-      const float zv = z[v];
-      d = expf(zv - m) * inv - ((uint32_t)v == y ? 1.0f : 0.0f);
-      d *= gs;
-      if (softcap > 0.f) {
-        const float tc = zv * ic;
-        d *= 1.0f - tc * tc;
+  auto grad = [&](float zv, float e, float inv, int v) {
+    float d = (e * inv - ((uint32_t)v == y ? 1.0f : 0.0f)) * gs;
+    if (softcap > 0.f) {
+      const float tc = zv * ic;
+      d *= 1.0f - tc * tc;
+    }
+    return d;
+  };
+  float m = -INFINITY, se = 0.f;
+  if constexpr (NV > 0) {
+    f32x4 zr[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int v = (i * CE_NT + threadIdx.x) * 4;
+      zr[i] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (v < V) zr[i] = *(const f32x4*)(z + v);
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) m = fmaxf(m, fmaxf(fmaxf(zr[i].x, zr[i].y), fmaxf(zr[i].z, zr[i].w)));
+    m = block_max<NW>(m, red);
+    f32x4 er[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int v = (i * CE_NT + threadIdx.x) * 4;
+      er[i] = f32x4{};
+      if (v < V) {
+        er[i].x = expf(zr[i].x - m);
+        er[i].y = expf(zr[i].y - m);
+        er[i].z = expf(zr[i].z - m);
+        er[i].w = expf(zr[i].w - m);
+        se += er[i].x + er[i].y + er[i].z + er[i].w;
       }
     }
-    o[v] = (f16)d;
+    se = block_sum<NW>(se, red);
+    const float inv = 1.0f / se;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int v = (i * CE_NT + threadIdx.x) * 4;
+      if (v < Vp) {
+        f16x4 h = {};
+        if (v < V) {
+          h.x = (f16)grad(zr[i].x, er[i].x, inv, v);
+          h.y = (f16)grad(zr[i].y, er[i].y, inv, v + 1);
+          h.z = (f16)grad(zr[i].z, er[i].z, inv, v + 2);
+          h.w = (f16)grad(zr[i].w, er[i].w, inv, v + 3);
+        }
+        *(f16x4*)(o + v) = h;
+      }
+    }
+  } else {
+    for (int v = threadIdx.x; v < V; v += CE_NT) m = fmaxf(m, z[v]);
+    m = block_max<NW>(m, red);
+    for (int v = threadIdx.x; v < V; v += CE_NT) se += expf(z[v] - m);
+    se = block_sum<NW>(se, red);
+    const float inv = 1.0f / se;
+    for (int v = threadIdx.x; v < Vp; v += CE_NT) o[v] = (f16)(v < V ? grad(z[v], expf(z[v] - m), inv, v) : 0.f);
   }
 }
 
@@ -145,8 +190,19 @@ hipError_t ce_backward(const float* logits, const uint32_t* tgt, int T, int V, i
                        float softcap, f16* dl, hipStream_t st) {
   if (T < 0 || V < 1 || Vp < V) return hipErrorInvalidValue;
   if (T == 0) return hipSuccess;
-  hipLaunchKernelGGL(ce_backward_kernel, dim3(T), dim3(256), 0, st, logits, tgt, V, Vp, gs, softcap,
-                     dl);
+  // registers while the row fits and its 16-byte accesses stay aligned (V and
+  // Vp multiples of 4 on 16-byte bases), the general form otherwise
+  const bool v4 = V % 4 == 0 && Vp % 4 == 0 && ((uintptr_t)logits & 15) == 0 && ((uintptr_t)dl & 7) == 0;
+  const int nv = v4 ? (Vp + 4 * CE_NT - 1) / (4 * CE_NT) : 0;
+#define HB_CE(n)                                                                                              \
+  hipLaunchKernelGGL(ce_backward_kernel<n>, dim3(T), dim3(CE_NT), 0, st, logits, tgt, V, Vp, gs, softcap, dl)
+  if (nv == 0 || nv > 16)
+    HB_CE(0);
+  else if (nv <= 4)
+    HB_CE(4);
+  else
+    HB_CE(16);
+#undef HB_CE
   return hipGetLastError();
 }
 
@@ -314,15 +370,16 @@ size_t rmsnorm_backward_part_floats(int dim) { return (size_t)NORM_PARTS * dim; 
 // the workgroup of position t returns unless t is the first occurrence of its
 // token; the first one sums the rows of every occurrence in position order
 // and adds the sum to the row of dE, so the result does not depend on
-// scheduling. Tokens are staged through LDS in chunks of EMB_CHUNK.
-constexpr int EMB_CHUNK = 4096;
+// scheduling. Each wave finds the later occurrences 64 positions at a time
+// with a ballot (one token per lane, read straight from L2); the positions
+// walked one by one took 139 us at 2048 tokens of 4096 features, this
+// EMB_BWD_US.
 constexpr int EMB_MAX_DIM = 8192;  // 8 float4 per thread
 __global__ __launch_bounds__(256) void embed_bwd_kernel(const float* __restrict__ dx,
                                                         const uint32_t* __restrict__ tok, int T,
                                                         int dim, int vocab,
                                                         float* __restrict__ dE) {
-  __shared__ uint32_t st[EMB_CHUNK];
-  const int t = blockIdx.x;
+  const int t = blockIdx.x, lane = threadIdx.x & 63;
   const uint32_t v = tok[t];
   if (v >= (uint32_t)vocab) return;  // the forward's embedding kernel reports it
   int dup = 0;
@@ -331,14 +388,13 @@ __global__ __launch_bounds__(256) void embed_bwd_kernel(const float* __restrict_
   f32x4 acc[EMB_MAX_DIM / 1024];
 #pragma unroll
   for (int k = 0; k < EMB_MAX_DIM / 1024; ++k) acc[k] = f32x4{};
-  for (int c0 = t; c0 < T; c0 += EMB_CHUNK) {
-    const int n = min(EMB_CHUNK, T - c0);
-    __syncthreads();
-    for (int u = threadIdx.x; u < n; u += 256) st[u] = tok[c0 + u];
-    __syncthreads();
-    for (int u = 0; u < n; ++u) {
-      if (st[u] != v) continue;
-      const float* row = dx + (size_t)(c0 + u) * dim;
+  for (int c0 = t; c0 < T; c0 += 64) {
+    const int u = c0 + lane;
+    uint64_t hits = __builtin_amdgcn_ballot_w64(u < T && tok[min(u, T - 1)] == v);
+    while (hits) {  // wave-uniform, the same in every wave
+      const int at = c0 + __builtin_ctzll(hits);
+      hits &= hits - 1;
+      const float* row = dx + (size_t)at * dim;
 #pragma unroll
       for (int k = 0; k < EMB_MAX_DIM / 1024; ++k) {
         const int i = k * 1024 + threadIdx.x * 4;

@@ -129,7 +129,7 @@ struct hb_model {
   size_t dbytes = 0;
   f16* t_embed = nullptr;
   bool dec_stale = true;
-  // split-K partial sums of the prefill residual GEMMs (gemm_splits)
+  // split-K partial sums of the residual and input-gradient GEMMs
   float* splitk = nullptr;
   size_t splitk_floats = 0;
   // Training state (transposed weights, kept activations, backward scratch),
@@ -417,14 +417,12 @@ int check_token_count(const hb_model_config& c, long B, long S) {
   return HB_OK;
 }
 
-// Scratch for a residual GEMM of this shape: grown on demand, empty when the
+// Scratch for a product of this shape in S splits: grown on demand, empty when the
 // shape does not split. A captured forward (forward_device_impl) reserves it
 // before the capture starts; growing it during a capture is refused
 // (HB_E_STATE), since it would allocate and synchronise inside the graph.
-int residual_scratch(hb_model* m, int N, int T, int K, GemmScratch& out, int wgs = 256) {
-  out = GemmScratch{m->splitk, m->splitk_floats, wgs};
-  bool wide;
-  const int S = std::max(gemm_splits(N, T, K, wgs), gemm_norm_splits(N, T, K, wgs, &wide));
+int split_scratch(hb_model* m, int N, int T, int S, GemmScratch& out) {
+  out = GemmScratch{m->splitk, m->splitk_floats};
   if (S <= 1) return HB_OK;
   const size_t need = (size_t)S * T * N;
   if (need > m->splitk_floats) {
@@ -437,8 +435,14 @@ int residual_scratch(hb_model* m, int N, int T, int K, GemmScratch& out, int wgs
     HIP_TRY(hipMalloc(&m->splitk, need * 4));
     m->splitk_floats = need;
   }
-  out = GemmScratch{m->splitk, m->splitk_floats, wgs};
+  out = GemmScratch{m->splitk, m->splitk_floats};
   return HB_OK;
+}
+int residual_scratch(hb_model* m, int N, int T, int K, GemmScratch& out) {
+  return split_scratch(m, N, T, std::max(gemm_splits(N, T, K), gemm_norm_splits(N, T, K)), out);
+}
+int store_scratch(hb_model* m, int N, int T, int K, GemmScratch& out) {
+  return split_scratch(m, N, T, gemm_store_splits(N, T, K), out);
 }
 
 bool weights_ready(hb_model* m) {
@@ -2242,7 +2246,7 @@ extern "C" int hb_op_wo_fwd_noalloc(hb_model* m, int layer, const void* attn, co
   float* sp = scratch_of(m->ctx->device);
   if (!sp) return fail(HB_E_STATE, "no-alloc scratch not set up on device %d", m->ctx->device);
   DeviceGuard g(m->ctx->device);
-  const GemmScratch so{sp, NOALLOC_SCRATCH_FLOATS, 256};
+  const GemmScratch so{sp, NOALLOC_SCRATCH_FLOATS};
   hipStream_t st = m->ctx->stream();
   // ordered after the previous use of the array unless the stream is being
   // captured (a graph's replays are ordered by whoever launches them)
@@ -2960,7 +2964,7 @@ int train_backward_impl(hb_model* m, hb_opt* o, int B, int S, float loss_scale) 
   HIP_TRY(ce_backward(ts->logits, ts->tgt, T, c.vocab, Vp, gs * f, ts->softcap, ts->dl, st));
   HIP_TRY(transpose_f16(ts->dl, T, c.vocab, Vp, 0, ts->dlT, Tp, 0, 1, st));
   GemmScratch se;
-  TRY(residual_scratch(m, d, T, Vp, se, 512));
+  TRY(store_scratch(m, d, T, Vp, se));
   HIP_TRY(gemm_store_split(ts->eT, ts->dl, d, T, Vp, ts->dtmp, &se, st, inv_f));
   HIP_TRY(transpose_f16(ts->xf, T, d, d, 0, ts->actT, Tp, 0, 1, st));
   HIP_TRY(gemm_wgrad(ts->actT, ts->dlT, d, c.vocab, Tp, g + o->embed_off, d, acc, st, inv_f));
@@ -2977,7 +2981,7 @@ int train_backward_impl(hb_model* m, hb_opt* o, int B, int S, float loss_scale) 
     HIP_TRY(gemm_silu_bwd(ts->w2T[l], ts->d16, h, T, d, EpiSiluBwd{A.h13, ts->dh, h}, st));
     HIP_TRY(transpose_f16(ts->dh, T, 2 * h, 2 * h, 0, ts->dhT, Tp, 0, 1, st));
     GemmScratch s13, sqkv;
-    TRY(residual_scratch(m, d, T, 2 * h, s13, 512));
+    TRY(store_scratch(m, d, T, 2 * h, s13));
     HIP_TRY(gemm_store_split(ts->w13T[l], ts->dh, d, T, 2 * h, ts->dtmp, &s13, st));
     HIP_TRY(transpose_f16(A.gate, T, h, h, 0, ts->actT, Tp, 0, 1, st));
     if (!(sq = slot(gemm_wgrad_max_tiles(h, d)))) return fail(HB_E_STATE, "gradient norm slots exhausted");
@@ -2999,7 +3003,7 @@ int train_backward_impl(hb_model* m, hb_opt* o, int B, int S, float loss_scale) 
     HIP_TRY(gemm_wgrad(ts->actT, ts->d16T, q, d, Tp, g + go.wo, q, acc, st, 1.0f, sq, &nt));
     ns += nt;
     TRY(attention_backward(m, A, B, S));
-    TRY(residual_scratch(m, d, T, qkv, sqkv, 512));
+    TRY(store_scratch(m, d, T, qkv, sqkv));
     HIP_TRY(gemm_store_split(ts->wqkvT[l], ts->dqkv, d, T, qkv, ts->dtmp, &sqkv, st));
     HIP_TRY(transpose_f16(A.xn, T, d, d, 0, ts->actT, Tp, 0, 1, st));
     if (!(sq = slot(gemm_wgrad_max_tiles(d, qkv)))) return fail(HB_E_STATE, "gradient norm slots exhausted");

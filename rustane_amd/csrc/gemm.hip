@@ -100,53 +100,114 @@ __global__ __launch_bounds__(256) void splitk_reduce_norm_kernel(const float* __
   }
 }
 
-int gemm_splits(int N, int T, int K, int wgs) {
+// Tile and split choice by predicted time. A launch of n workgroups (tiles x
+// splits) takes n / 256 rounds of the 256 CUs, a partly filled last round
+// counting 0.65 + 0.35 x its fill (its tiles run faster with fewer
+// neighbours), of slice_us per 64-wide K slice plus tile_us per tile
+// (prologue and epilogue). The constants are fitted to launches at 45 to 4096
+// tokens of the 7B, 5B and 600M shapes with K = 512 to 11008: the choice is
+// the fastest measured tile in 15 of 16 of them and 2% off in the other. For
+// instance, us per tile 256x256 / 192x256 / 128x256 / 192x128 / 128x128 /
+// 64x128: 12288 x 4096 x 4096 320 / 328 / 350 / 372 / 445 / 575; 22016 x 512 x
+// 4096 87 / 78 / 104 / 90 / 106 / 133; 22016 x 45 x 4096 69 / 55 / 46 / 43 / 31 /
+// 42. 192x128 and 128x128 workgroups run two to a CU.
+const GemmTile GEMM_TILES[6] = {{256, 256, 1.43f, 10.f}, {192, 256, 1.11f, 8.f},  {128, 256, 0.83f, 6.5f},
+                                {192, 128, 0.64f, 7.f},  {128, 128, 0.49f, 5.f},  {64, 128, 0.34f, 4.f}};
+static constexpr int GEMM_CUS = 256;  // MI355X compute units
+
+GemmChoice gemm_tile(int N, int T, int K, int S, float* us) {
+  const int kq = (K / 64 + S - 1) / S;
+  GemmChoice best{0, S};
+  float best_us = INFINITY;
+  for (int i = 0; i < 6; ++i) {
+    const GemmTile& g = GEMM_TILES[i];
+    const long n = ntiles(N, T, g.ft, g.tt) * S;
+    const float fill = (float)(n % GEMM_CUS) / GEMM_CUS;
+    const float rounds = (float)(n / GEMM_CUS) + (fill > 0.f ? 0.65f + 0.35f * fill : 0.f);
+    const float t = rounds * ((float)kq * g.slice_us + g.tile_us);
+    if (t < best_us) {
+      best_us = t;
+      best.tile = i;
+    }
+  }
+  if (us) *us = best_us;
+  return best;
+}
+
+// Long-K residual projections with few output tiles (Wo and W2 at 512 tokens:
+// 128 tiles of 128x128) split K over up to GEMM_MAX_SPLITS ranges of >= 8
+// slices so that ~256 workgroups run; the partials go through the caller's
+// scratch and splitk_reduce applies the epilogue. The number of splits fixes
+// the order of the sums, the tile (gemm_tile) does not. K from 1024 splits too
+// (600M shape, Wo with K = 1536 at 512 tokens: 96 workgroups of 64x128 unsplit,
+// 144 of 128x128 in 3 splits; the batch-1 forward 2.28 -> 2.16 ms).
+int gemm_splits(int N, int T, int K) {
   const long t = ntiles(N, T, 128, 128);
   const int nk = K / 64;
-  if (t >= wgs || nk < 16) return 1;
-  int S = (int)std::min<long>(GEMM_MAX_SPLITS, wgs / t);
+  if (t >= GEMM_CUS || nk < 16) return 1;
+  int S = (int)std::min<long>(GEMM_MAX_SPLITS, GEMM_CUS / t);
   S = std::min(S, nk / 8);
   return S >= 2 ? S : 1;
 }
 
 // The residual + RMSNorm projections (gemm_residual_norm): a long reduction
-// (K >= 2N) whose 128x256 tiles in S splits fill the wgs workgroups exactly
-// runs on those tiles (7B W2 at 512 tokens: 64 tiles x 4 splits instead of
-// 128 of 128x128 x 2; GEMM alone 54 -> 45.5 us: the wider tile's main loop
-// outweighs the reduce reading 4 partials instead of 2; Wo, K = N, gains less).
-// Otherwise gemm_splits on 128x128 tiles. *wide tells which.
-int gemm_norm_splits(int N, int T, int K, int wgs, bool* wide) {
-  *wide = false;
-  const int S = gemm_splits(N, T, K, wgs);
+// (K >= 2N) whose 128x256 tiles in S splits fill the CUs exactly takes those
+// (7B W2 at 512 tokens: 64 tiles x 4 splits instead of 128 of 128x128 x 2;
+// GEMM alone 54 -> 45.5 us: the wider tile's main loop outweighs the reduce
+// reading 4 partials instead of 2; Wo, K = N, gains less).
+int gemm_norm_splits(int N, int T, int K) {
+  const int S = gemm_splits(N, T, K);
   if (S <= 1 || K < 2 * N) return S;
-  const long t = ntiles(N, T, 128, 256);
-  if (t <= 0 || wgs % t) return S;
-  const int Sw = (int)(wgs / t);
-  if (Sw < 2 || Sw > GEMM_MAX_SPLITS || Sw * 8 > K / 64) return S;
-  *wide = true;
-  return Sw;
+  const long t = ntiles(N, T, 256, 128);
+  if (t <= 0 || GEMM_CUS % t) return S;
+  const int Sw = (int)(GEMM_CUS / t);
+  return Sw < 2 || Sw > GEMM_MAX_SPLITS || Sw * 8 > K / 64 ? S : Sw;
+}
+
+// The input-gradient products (gemm_store_split): any number of splits of >= 8
+// slices, by predicted time: REDUCE_US for the reduction's launch and
+// (splits + 2) x T x N floats through memory at ~4.5 TB/s. N = 2560 at 2048
+// tokens has 80 tiles of 256x256; K = 13824 and 32000 take them in 3 splits
+// (all five products of a layer and head 186 us on average unsplit on 192x128
+// tiles, 158 with the reduction).
+int gemm_store_splits(int N, int T, int K) {
+  constexpr float REDUCE_US = 3.f, US_PER_BYTE = 1.f / 4.5e6f;
+  const int nk = K / 64;
+  const size_t TN = (size_t)T * N;
+  int best = 1;
+  float best_us = INFINITY;
+  for (int S = 1; S <= GEMM_MAX_SPLITS && (S == 1 || nk >= 8 * S); ++S) {
+    if ((S - 1) * ((nk + S - 1) / S) >= nk) continue;
+    float us;
+    (void)gemm_tile(N, T, K, S, &us);
+    if (S > 1) us += REDUCE_US + (float)(S + 2) * 4.f * (float)TN * US_PER_BYTE;
+    if (us < best_us) {
+      best_us = us;
+      best = S;
+    }
+  }
+  return best;
 }
 
 hipError_t gemm_store(const f16* W, const f16* X, int N, int T, int K, float* C, hipStream_t st) {
-  return launch_gemm(W, X, N, T, K, EpiStore{C, N}, nullptr, st);
+  return launch_gemm(W, X, N, T, K, EpiStore{C, N}, st);
 }
 hipError_t gemm_residual(const f16* W, const f16* X, int N, int T, int K, const EpiResidual& e,
                          const GemmScratch* scr, hipStream_t st, int kw) {
-  return launch_gemm(W, X, N, T, K, e, scr, st, kw);
+  return launch_split_gemm(W, X, N, T, K, e, scr ? gemm_splits(N, T, K) : 1, scr, st, kw);
 }
 hipError_t gemm_residual_norm(const f16* W, const f16* X, int N, int T, int K, const EpiResidual& e,
                               const NormOut& no, const GemmScratch* scr, hipStream_t st, int kw,
                               hipEvent_t mid) {
   if (e.ld != N) return hipErrorInvalidValue;
-  bool wide = false;
-  const int S = scr ? gemm_norm_splits(N, T, K, scr->wgs, &wide) : 1;
+  if (!gemm_fits(N, T, K)) return hipErrorInvalidValue;
+  const GemmChoice c = gemm_tile(N, T, K, scr ? gemm_norm_splits(N, T, K) : 1);
+  const int S = c.splits;
   hipError_t err2 = hipSuccess;
   if (S > 1) {
     const size_t stride = (size_t)T * N;
-    if (!scr->p || (size_t)S * stride > scr->floats || (long)N * K >= (1L << 31)) return hipErrorInvalidValue;
-    const hipError_t err =
-        wide ? launch_tile<128, 256>(W, X, N, T, K, EpiSplit{scr->p, N, stride}, st, S, kw)
-             : launch_tile<128, 128>(W, X, N, T, K, EpiSplit{scr->p, N, stride}, st, S, kw);
+    if (!scr->p || (size_t)S * stride > scr->floats) return hipErrorInvalidValue;
+    const hipError_t err = launch_choice(c, W, X, N, T, K, EpiSplit{scr->p, N, stride}, st, kw);
     if (err != hipSuccess) return err;
     if (mid && (err2 = hipEventRecord(mid, st)) != hipSuccess) return err2;
     // 1..8: whole multiples of 1024; 9..16: ragged, ceil(N / 1024) = 1..8
@@ -167,7 +228,7 @@ hipError_t gemm_residual_norm(const f16* W, const f16* X, int N, int T, int K, c
     }
     return hipGetLastError();
   }
-  const hipError_t err = launch_gemm(W, X, N, T, K, e, nullptr, st, kw);
+  const hipError_t err = launch_choice(c, W, X, N, T, K, e, st, kw);
   if (err != hipSuccess) return err;
   if (mid && (err2 = hipEventRecord(mid, st)) != hipSuccess) return err2;
   return rmsnorm(e.out, N, no.gamma, T, N, no.eps, no.xn, nullptr, st, no.split);
@@ -175,7 +236,7 @@ hipError_t gemm_residual_norm(const f16* W, const f16* X, int N, int T, int K, c
 // ---- training ----
 hipError_t gemm_store_split(const f16* W, const f16* X, int N, int T, int K, float* C,
                             const GemmScratch* scr, hipStream_t st, float scale) {
-  return launch_gemm(W, X, N, T, K, EpiStore{C, N, scale}, scr, st);
+  return launch_split_gemm(W, X, N, T, K, EpiStore{C, N, scale}, scr ? gemm_store_splits(N, T, K) : 1, scr, st);
 }
 
 }  // namespace hb

@@ -52,82 +52,60 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   }
 }
 
-// Tile choice: maximise (relative per-tile throughput) x (tiles per CU-round
-// of the 256 CUs). Relative throughputs are measured on MI355X with whole
-// rounds of tiles (12288 x 4096 x 4096, us: 256x256 320, 192x256 328, 128x256
-// 350, 192x128 372 on gemm_nt_kernel; 128x128 444, 64x128 575 on
-// gemm_nt_kernel_reg). At 512 tokens this picks 192x256 for W1|W3 (230
-// tiles), 192x128 for QKV (256 tiles) and 256x256 for the logits; at
-// 4096 tokens 256x256 throughout.
-//
-// Long-K problems with few output tiles (Wo and W2 at 512 tokens: 128 tiles of
-// 128x128) instead split K over up to GEMM_MAX_SPLITS ranges of >= 8 slices so
-// that ~256 workgroups run; the partials go through the caller's scratch and
-// splitk_reduce applies the epilogue. Measured GEMM time at 512 tokens, 7B
-// shapes: Wo 23.4 us (128x128 x 2 splits; 128x256 unsplit 29.2); W2 54 us
-// (128x128 x 2) against 45.5 us (128x256 x 4). Two splits halve the
-// partial-sum traffic of the reduce; the long-K residual + norm projections
-// (W2) still take 128x256 x 4 (gemm_norm_splits), where the GEMM's gain
-// outweighs the larger reduce.
-// K from 1024 splits too (600M shape, Wo with K = 1536 at 512 tokens: 96
-// workgroups of 64x128 unsplit, 144 of 128x128 in 3 splits; the batch-1
-// forward 2.28 -> 2.16 ms).
-constexpr int GEMM_CUS = 256;  // MI355X compute units
+// A tile (index into GEMM_TILES, gemm.hip) and a number of K splits.
+struct GemmChoice {
+  int tile, splits;
+};
+struct GemmTile {
+  int ft, tt;
+  float slice_us, tile_us;
+};
+extern const GemmTile GEMM_TILES[6];
+// The fastest tile of a product in `splits` K splits, and its predicted time.
+GemmChoice gemm_tile(int N, int T, int K, int splits, float* us = nullptr);
+
+template <class Epi>
+static hipError_t launch_choice(GemmChoice c, const f16* W, const f16* X, int N, int T, int K, const Epi& epi,
+                                hipStream_t st, int kw) {
+  switch (c.tile) {
+    case 0: return launch_tile<256, 256>(W, X, N, T, K, epi, st, c.splits, kw);
+    case 1: return launch_tile<192, 256>(W, X, N, T, K, epi, st, c.splits, kw);
+    case 2: return launch_tile<128, 256>(W, X, N, T, K, epi, st, c.splits, kw);
+    case 3: return launch_tile<192, 128>(W, X, N, T, K, epi, st, c.splits, kw);
+    case 4: return launch_tile<128, 128>(W, X, N, T, K, epi, st, c.splits, kw);
+    default: return launch_tile<64, 128>(W, X, N, T, K, epi, st, c.splits, kw);
+  }
+}
 inline long ntiles(int N, int T, int ft, int tt) { return (long)((N + ft - 1) / ft) * ((T + tt - 1) / tt); }
 
-// tiles (nullable): receives the number of output tiles launched.
+inline bool gemm_fits(int N, int T, int K) { return (long)N * K < (1L << 31) && (long)T * K < (1L << 31); }
+
+// Unsplit product; tiles (nullable) receives the number of output tiles.
 template <class Epi>
 static hipError_t launch_gemm(const f16* W, const f16* X, int N, int T, int K, const Epi& epi,
-                              const GemmScratch* scr, hipStream_t st, int kw = 0, int* tiles = nullptr) {
-  if ((long)N * K >= (1L << 31) || (long)T * K >= (1L << 31)) return hipErrorInvalidValue;
-  const int S = scr ? gemm_splits(N, T, K, scr->wgs) : 1;
-  if constexpr (!EpiSumSq<Epi>::value) {
-    if (S > 1) {
-      const size_t stride = (size_t)T * N;
-      if (!scr->p || (size_t)S * stride > scr->floats) return hipErrorInvalidValue;
-      const hipError_t e = launch_tile<128, 128>(W, X, N, T, K, EpiSplit{scr->p, N, stride}, st, S, kw);
-      if (e != hipSuccess) return e;
-      const size_t n4 = stride / 4;
-      const int grid = (int)std::min<size_t>((n4 + 255) / 256, 4096);
-      hipLaunchKernelGGL((splitk_reduce_kernel<Epi>), dim3(grid), dim3(256), 0, st, scr->p, S, T, N,
-                         stride, epi);
-      return hipGetLastError();
-    }
-  }
-  // rel: throughput per CU of each tile shape with every CU busy (time per
-  // full round of workgroups per tile area, 256x256 = 1); the score is the
-  // output area over the rounds' time, where a partly filled last round counts
-  // 0.4 + 0.6 x its fill (its tiles run faster with fewer neighbours: fitted
-  // to the measured 7B launches at 512 and 4096 tokens). Area past N or T
-  // earns nothing: 45 tokens take 128x128 tiles (22016 x 45 x 4096: 31.4 us),
-  // not 128x256 (45.7 us).
-  struct Cand {
-    int ft, tt;
-    float rel;
-  };
-  static constexpr Cand cands[] = {{256, 256, 1.00f}, {192, 256, 0.97f}, {128, 256, 0.91f},
-                                   {192, 128, 0.86f}, {128, 128, 0.73f}, {64, 128, 0.53f}};
-  int best = 0;
-  float best_score = -1.f;
-  for (int i = 0; i < (int)(sizeof(cands) / sizeof(cands[0])); ++i) {
-    const long n = ntiles(N, T, cands[i].ft, cands[i].tt);
-    const float fill = (float)(n % GEMM_CUS) / GEMM_CUS;
-    const float rounds = (float)(n / GEMM_CUS) + (fill > 0.f ? 0.4f + 0.6f * fill : 0.f);
-    const float score = cands[i].rel * (float)N * (float)T / (rounds * (float)(cands[i].ft * cands[i].tt));
-    if (score > best_score * 1.000001f) {
-      best_score = score;
-      best = i;
-    }
-  }
-  if (tiles) *tiles = (int)ntiles(N, T, cands[best].ft, cands[best].tt);
-  switch (best) {
-    case 0: return launch_tile<256, 256>(W, X, N, T, K, epi, st, 1, kw);
-    case 1: return launch_tile<192, 256>(W, X, N, T, K, epi, st, 1, kw);
-    case 2: return launch_tile<128, 256>(W, X, N, T, K, epi, st, 1, kw);
-    case 3: return launch_tile<192, 128>(W, X, N, T, K, epi, st, 1, kw);
-    case 4: return launch_tile<128, 128>(W, X, N, T, K, epi, st, 1, kw);
-    default: return launch_tile<64, 128>(W, X, N, T, K, epi, st, 1, kw);
-  }
+                              hipStream_t st, int kw = 0, int* tiles = nullptr) {
+  if (!gemm_fits(N, T, K)) return hipErrorInvalidValue;
+  const GemmChoice c = gemm_tile(N, T, K, 1);
+  if (tiles) *tiles = (int)ntiles(N, T, GEMM_TILES[c.tile].ft, GEMM_TILES[c.tile].tt);
+  return launch_choice(c, W, X, N, T, K, epi, st, kw);
+}
+
+// Product in S splits of K through the caller's scratch.
+template <class Epi>
+static hipError_t launch_split_gemm(const f16* W, const f16* X, int N, int T, int K, const Epi& epi,
+                                    int S, const GemmScratch* scr, hipStream_t st, int kw = 0) {
+  if (!gemm_fits(N, T, K)) return hipErrorInvalidValue;
+  const GemmChoice c = gemm_tile(N, T, K, S);
+  if (c.splits == 1) return launch_choice(c, W, X, N, T, K, epi, st, kw);
+  const size_t stride = (size_t)T * N;
+  if (!scr->p || c.splits * stride > scr->floats) return hipErrorInvalidValue;
+  const hipError_t e = launch_choice(c, W, X, N, T, K, EpiSplit{scr->p, N, stride}, st, kw);
+  if (e != hipSuccess) return e;
+  const size_t n4 = stride / 4;
+  const int grid = (int)std::min<size_t>((n4 + 255) / 256, 4096);
+  hipLaunchKernelGGL((splitk_reduce_kernel<Epi>), dim3(grid), dim3(256), 0, st, scr->p, c.splits, T, N,
+                     stride, epi);
+  return hipGetLastError();
 }
 
 }  // namespace hb

@@ -9,7 +9,7 @@ hipError_t gemm_qkv(const f16* W, const f16* X, int N, int T, int K, const EpiQK
   auto run = [&](auto mode) {
     EpiQKVAt<false, decltype(mode)::value> ep(e);
     ep.prepare();
-    return launch_gemm(W, X, N, T, K, ep, nullptr, st, kw);
+    return launch_gemm(W, X, N, T, K, ep, st, kw);
   };
   switch (e.mode()) {
     case EpiQKV::PLAIN: return run(std::integral_constant<int, EpiQKV::PLAIN>{});

@@ -6,19 +6,19 @@
 namespace hb {
 
 // ---- prefill GEMM (gemm.hip, gemm_qkv.hip, gemm_ffn.hip, gemm_train.hip) ----
-// Scratch for split-K partial sums (fp32); see gemm_splits.
+// Scratch for split-K partial sums (fp32), grown by the caller.
 struct GemmScratch {
   float* p;
   size_t floats;
-  int wgs = 256;  // workgroups the split count aims for (gemm_splits)
 };
 constexpr int GEMM_MAX_SPLITS = 8;
 // Number of K splits the residual GEMM uses for this shape when given scratch
-// (1 = none), aiming at wgs workgroups; it needs splits * T * N floats.
-int gemm_splits(int N, int T, int K, int wgs = 256);
-// The same for gemm_residual_norm, which may use 128x256 tiles (*wide) for
-// long reductions; it needs splits * T * N floats too.
-int gemm_norm_splits(int N, int T, int K, int wgs, bool* wide);
+// (1 = none); it needs splits * T * N floats.
+int gemm_splits(int N, int T, int K);
+// The same for gemm_residual_norm, which splits long reductions further.
+int gemm_norm_splits(int N, int T, int K);
+// The same for gemm_store_split.
+int gemm_store_splits(int N, int T, int K);
 hipError_t gemm_store(const f16* W, const f16* X, int N, int T, int K, float* C, hipStream_t st);
 // kw (the residual, SwiGLU and QKV projections): 0 for plain X rows of K
 // halves; for split X rows (common.hpp) K = 2 * kw with kw the weights' row
@@ -48,7 +48,7 @@ hipError_t gemm_qkv(const f16* W, const f16* X, int N, int T, int K, const EpiQK
 // Training products (the epilogues are documented in epilogue.hpp). All take
 // K % 64 == 0; token-dimension (K = tokens) operands are zero-padded to it.
 // C = X W^T (fp32 store), split over K into scr when the shape leaves CUs idle
-// (gemm_splits), as the residual GEMMs are.
+// (gemm_store_splits).
 hipError_t gemm_store_split(const f16* W, const f16* X, int N, int T, int K, float* C,
                             const GemmScratch* scr, hipStream_t st, float scale = 1.0f);
 // Weight gradient g[t, f] (+)= sum_k X[t,k] W[f,k]: accumulate (EpiAccum) or,

@@ -115,6 +115,25 @@ def test_tiny_mha_full_sequence():
     st.close()
 
 
+@pytest.mark.parametrize("vocab,S", [
+    (8256, 70),    # the logits row of the CE backward in registers, its last chunks past the row
+    (33024, 12),   # wider than the registers hold: the general form
+    (64, 130),     # every token many times, further apart than one ballot of the embedding backward
+])
+def test_head_kernels_at_their_size_limits(vocab, S):
+    cfg = tiny_config(vocab=vocab, seq=S)
+    _, st, *_ = _run_case(cfg, 2, S, seed=31, softcap=15.0 if vocab == 8256 else 0.0)
+    st.close()
+
+
+def test_input_gradients_split_over_k():
+    """Few tokens and a long reduction (K = vocab = 8192, 2 * hidden = 4096):
+    the input-gradient products run in several K splits."""
+    cfg = tiny_config(dim=256, hidden=2048, heads=4, vocab=8192, seq=96, nlayers=1)
+    _, st, *_ = _run_case(cfg, 1, 96, seed=33)
+    st.close()
+
+
 def test_long_sequence_attention_kernels_hd128():
     """Enough (query block, head, sequence) groups -- 16 sequences of 500 at 8
     heads of 128 -- that the attention kernels take the variants the 7B shape
