@@ -11,9 +11,17 @@
 // a row tile [32][hd] is read as A-operand rows in swap23 slot order (chunk c
 // of row r at r*NCH + (c ^ (swap23(r) % NCH))), so the 8 accumulator
 // registers 8j..8j+7 of lane half h2 hold the consecutive rows 16j+8h2..+7
-// and serve directly as a B operand; a column tile [hd][32] (chunk c of row e
-// at e*4 + (c ^ ((e >> 2) & 3))) gives A fragments of one hd row and 8
-// consecutive keys or queries.
+// and serve directly as a B operand. The same tile also gives the transposed
+// A operand (one feature, 8 consecutive rows) through ds_read_b64_tr_b16
+// (tr_frag), so no transposed copies exist in memory or LDS.
+//
+// Tiles go from global memory straight into LDS (dma_1k) one or two
+// iterations ahead, with one barrier per iteration; a workgroup is 4 waves of
+// at most 256 registers, two workgroups to a CU, so that one's softmax and
+// waits run under the other's MFMAs. The predecessors (register-staged
+// double-buffered tiles, transposed copies, one workgroup of 4 waves per CU)
+// spent most of an iteration waiting: 20 heads x 2048 of 128, us: dQ 344 ->
+// 154, dK/dV 336 -> 121; 32 heads x 4 x 512, 70 -> 64 and 99 -> 51.
 //
 // attn_bwd_dq_kernel, per (PQ query blocks, head, sequence), PQ x PK waves
 // (PK key parts): S^T = K Q^T and dP^T = V dO^T per key block, two passes
@@ -60,26 +68,84 @@ HB_DEV void store_grad4(const AttnBwd& p, int b, int s, int col, int f0, f32x4 v
   p.dqkvT[(size_t)(col + 3) * p.tld + tok] = h.w;
 }
 
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// Transposed A fragments of a row tile. ds_read_b64_tr_b16: in each group of
+// 16 lanes, lane s supplies 4 halves of its own address and lane i receives,
+// as element e, half i%4 of lane 4e + i/4. With lane s at row base + s/4,
+// features F + 4(s%4)..+3, lane i gets feature F + i of rows base..base+3.
+// The fragment (m, j) of lane (h2, li) is feature m*32 + li of rows 16j + 8h2
+// .. +7: two reads. The tile's chunk swizzle enters through the two lane
+// bases (m even, odd); everything else is an immediate offset.
 template <int HD>
-HB_DEV int row_chunk(int r, int c) {  // row tile: chunk c of row r
-  constexpr int NCH = HD / 8;
-  return r * NCH + (c ^ (swap23(r) % NCH));
-}
-HB_DEV int col_chunk(int e, int c) { return e * 4 + (c ^ ((e >> 2) & 3)); }  // column tile
+struct TrFrag {
+  static constexpr int NCH = HD / 8;
+  int base[2];
+  HB_DEV explicit TrFrag(int lane) {
+    const int s = lane & 15, g = lane >> 4, h2 = lane >> 5;
+#pragma unroll
+    for (int mm = 0; mm < 2; ++mm) {
+      const int c = mm * 4 + 2 * (g & 1) + ((s & 3) >> 1), x = (4 * h2 + (s >> 2)) % NCH;
+      base[mm] = ((8 * h2 + (s >> 2)) * NCH + (c ^ x)) * 8 + 4 * (s & 1);
+    }
+  }
+  HB_DEV f16x8 read(const f16x8* tile, int m, int j) const {
+    const f16* t = (const f16*)tile + base[m & 1];
+    s16x4 v[2];
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {
+      const int off = (16 * j + 4 * hh) * NCH * 8 + (NCH == 16 ? ((hh ^ (m >> 1)) & 1) * 64 : 0);
+      v[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (__attribute__((address_space(3))) s16x4*)(__attribute__((address_space(3))) void*)(t + off));
+    }
+    const auto w = __builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(f16x8, w);
+  }
+};
+
+// Copies of one iteration's tiles by PW waves: tile t = kind * PARTS + part is
+// 32 rows of HD halves at base[kind] + row0(part) * HD, NI instructions of
+// 1 KB per wave.
+template <int HD, int PW, int PARTS>
+struct TileDma {
+  static constexpr int NCH = HD / 8, IPT = HD / 16;  // instructions per tile
+  static constexpr int NI = 2 * PARTS * IPT / PW;
+  static constexpr uint32_t BYTES = 2 * PARTS * HD * 64;
+  static_assert(IPT % PW == 0, "an instruction slot belongs to one tile");
+  uint32_t voff[IPT / PW];
+  uint32_t lds;
+  i32x4 rs[2];
+  HB_DEV TileDma(const f16* b0, const f16* b1, uint32_t lds0, int wave, int lane) : lds(lds0 + wave * 1024) {
+    rs[0] = dma_rsrc(b0);
+    rs[1] = dma_rsrc(b1);
+#pragma unroll
+    for (int u = 0; u < IPT / PW; ++u) {
+      const int row = (wave + PW * u) * (64 / NCH) + lane / NCH;
+      voff[u] = (uint32_t)(row * HD + ((lane % NCH) ^ (swap23(row) % NCH)) * 8) * 2u;
+    }
+  }
+  // row0: (kind, part) -> first row, wave-uniform
+  template <class F>
+  HB_DEV void issue(int buf, F&& row0) const {
+#pragma unroll
+    for (int u = 0; u < NI; ++u) {
+      const int tile = u * PW / IPT, kind = tile / PARTS, part = tile % PARTS;
+      dma_1k(lds + buf * BYTES + u * PW * 1024, voff[u % (IPT / PW)], rs[kind],
+             (uint32_t)row0(part) * (uint32_t)(HD * 2));
+    }
+  }
+};
 
 }  // namespace
 
 template <int HD, int PQ, int PK>
-__global__ __launch_bounds__(PQ * PK * 64, 1) void attn_bwd_dq_kernel(AttnBwd p) {
+__global__ __launch_bounds__(PQ * PK * 64, 2) void attn_bwd_dq_kernel(AttnBwd p) {
   constexpr int PW = PQ * PK;  // waves: query blocks x key parts
   constexpr int KS = HD / 16, MB = HD / 32, NCH = HD / 8, KT8 = 4 * HD;
-  constexpr int NKIND = 3;  // K rows, V rows, K^T columns
-  constexpr int NLD = NKIND * PK * KT8 / (PW * 64);
-  static_assert(NLD * PW * 64 == NKIND * PK * KT8, "loader coverage");
-  // two tile buffers: iteration n computes from buffer n & 1 while the tiles
-  // of n + 1 go into the other one (one barrier per iteration)
-  constexpr int NTILE = NKIND * PK * KT8, NMERGE = PK == 2 ? PQ * MB * 16 * 64 * 4 / 16 : 0;
-  __shared__ f16x8 s_t[2 * NTILE > NMERGE ? 2 * NTILE : NMERGE];
+  constexpr int NB = PK == 1 ? 3 : 2;  // tile buffers: K and V rows of PK key blocks each
+  using Dma = TileDma<HD, PW, PK>;
+  constexpr int NTILE = 2 * PK * KT8, NMERGE = PK == 2 ? PQ * MB * 16 * 64 * 4 / 16 : 0;
+  __shared__ f16x8 s_t[NB * NTILE > NMERGE ? NB * NTILE : NMERGE];
   __shared__ float s_d[PQ][64];
 
   const int tid = threadIdx.x, lane = tid & 63, h2 = lane >> 5, li = lane & 31;
@@ -110,51 +176,32 @@ __global__ __launch_bounds__(PQ * PK * 64, 1) void attn_bwd_dq_kernel(AttnBwd p)
     if (qi < p.S) L2 = p.lse[qrow + qi];
   }
 
-  const f16* kz = p.k + (size_t)z * p.Sp * HD;
-  const f16* vz = p.v + (size_t)z * p.Sp * HD;
-  const f16* ktz = p.kT + (size_t)z * HD * p.Sp;
-  f16x8 reg[NLD];
-  auto gload = [&](int n, bool with_t) {
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int x = i * PW * 64 + tid, tile = x / KT8, y = x % KT8;
-      const int kind = tile / PK, kb = min(n * PK + tile % PK, nkb - 1);
-      if (kind < 2) {
-        const f16* base = kind == 0 ? kz : vz;
-        reg[i] = *(const f16x8*)(base + ((size_t)kb * 32 + y / NCH) * HD + (y % NCH) * 8);
-      } else if (with_t) {
-        reg[i] = *(const f16x8*)(ktz + (size_t)(y >> 2) * p.Sp + kb * 32 + (y & 3) * 8);
-      }
-    }
-  };
-  auto lstore = [&](int buf, bool with_t) {
-    f16x8* st = s_t + buf * NTILE;
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int x = i * PW * 64 + tid, tile = x / KT8, y = x % KT8;
-      if (tile / PK < 2)
-        st[tile * KT8 + row_chunk<HD>(y / NCH, y % NCH)] = reg[i];
-      else if (with_t)
-        st[tile * KT8 + col_chunk(y >> 2, y & 3)] = reg[i];
-    }
-  };
-
+  const Dma dma(p.k + (size_t)z * p.Sp * HD, p.v + (size_t)z * p.Sp * HD, lds_addr(s_t), wave, lane);
+  const TrFrag<HD> tr(lane);
   const float sl2 = p.scale * HB_LOG2E;
   const int krow = swap23(li);
   const int niter = (nkb + PK - 1) / PK;
-  // the key loop of one pass: body(n, tile buffer) on every iteration's tiles
-  auto keyloop = [&](bool with_t, auto&& body) {
-    gload(0, with_t);
-    lstore(0, with_t);
-    if (niter > 1) gload(1, with_t);
-    lds_barrier();
+  auto issue = [&](int n, int buf) {
+    dma.issue(buf, [&](int part) { return min(n * PK + part, nkb - 1) * 32; });
+  };
+  // the key loop of one pass: body(n, tiles) on every iteration's tiles, the
+  // copies NB - 1 iterations ahead. The barrier of iteration n follows every
+  // wave's wait for its own copies of n and its last read of n - 1, whose
+  // buffer the new copies go into.
+  auto keyloop = [&](auto&& body) {
+    raw_barrier();  // the other waves are done with LDS
+    issue(0, 0);
+    if (NB == 3 && niter > 1) issue(1, 1);
+    int buf = 0;
     for (int n = 0; n < niter; ++n) {
-      body(n, s_t + (n & 1) * NTILE);
-      if (n + 1 < niter) {
-        lstore((n + 1) & 1, with_t);  // that buffer was last read in iteration n - 1
-        if (n + 2 < niter) gload(n + 2, with_t);
-      }
-      lds_barrier();
+      if (NB == 3 && n + 1 < niter)
+        dma_wait<Dma::NI>();
+      else
+        dma_wait<0>();
+      raw_barrier();
+      if (n + NB - 1 < niter) issue(n + NB - 1, buf == 0 ? NB - 1 : buf - 1);
+      body(n, s_t + buf * NTILE);
+      buf = buf == NB - 1 ? 0 : buf + 1;
     }
   };
   // S^T and dP^T of key block kb against this wave's queries; s becomes P
@@ -163,23 +210,33 @@ __global__ __launch_bounds__(PQ * PK * 64, 1) void attn_bwd_dq_kernel(AttnBwd p)
     const f16x8* sv = st + (PK + kh) * KT8;
     s = f32x16{};
     dp = f32x16{};
+    f16x8 kf[KS];
 #pragma unroll
-    for (int j = 0; j < KS; ++j) {
-      const int ko = krow * NCH + ((2 * j + h2) ^ (li % NCH));
-      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sk[ko], qf[j], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv[ko], df[j], dp, 0, 0, 0);
-    }
-    // masked entries get exp2(-inf) = 0: a select on the argument, no branch
+    for (int j = 0; j < KS; ++j) kf[j] = sk[krow * NCH + ((2 * j + h2) ^ (li % NCH))];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int key = kb * 32 + swap23(8 * (r >> 2) + 4 * h2 + (r & 3));
-      s[r] = exp2f((qok && key <= qi) ? s[r] * sl2 - L2 : -INFINITY);
+    for (int j = 0; j < KS; ++j) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[j], qf[j], s, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < KS; ++j) kf[j] = sv[krow * NCH + ((2 * j + h2) ^ (li % NCH))];
+#pragma unroll
+    for (int j = 0; j < KS; ++j) dp = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[j], df[j], dp, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = s[r] * sl2 - L2;
+    // keys after the query exist in its diagonal block only (padding keys
+    // come after every valid query); queries past S are never stored
+    if (kb == qb) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (kb * 32 + swap23(8 * (r >> 2) + 4 * h2 + (r & 3)) > qi) s[r] = -INFINITY;
     }
+    // v_exp_f32 itself: what exp2f's range scaling would add, results below
+    // 2^-126, is 0 in every use
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(s[r]);
   };
 
   // pass 1: D = rowsum(P * dP) over this wave's key half, then over both
   float dsum = 0.f;
-  keyloop(false, [&](int n, const f16x8* st) {
+  keyloop([&](int n, const f16x8* st) {
     const int kb = n * PK + kh;
     if (!active || kb > qb) return;  // wave-uniform
     f32x16 s, dp;
@@ -204,30 +261,29 @@ __global__ __launch_bounds__(PQ * PK * 64, 1) void attn_bwd_dq_kernel(AttnBwd p)
   f32x16 o[MB];
 #pragma unroll
   for (int m = 0; m < MB; ++m) o[m] = f32x16{};
-  keyloop(true, [&](int n, const f16x8* st) {
+  keyloop([&](int n, const f16x8* st) {
     const int kb = n * PK + kh;
     if (!active || kb > qb) return;
     f32x16 s, dp;
     block(st, kb, s, dp);
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = s[r] * (dp[r] - D) * p.scale;
-    const f16x8* skt = st + (2 * PK + kh) * KT8;
+    const f16x8* sk = st + kh * KT8;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       f16x8 db;
 #pragma unroll
       for (int i = 0; i < 8; ++i) db[i] = (f16)s[8 * j + i];
 #pragma unroll
-      for (int m = 0; m < MB; ++m) {
-        const int e = m * 32 + li;
-        o[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(skt[col_chunk(e, 2 * j + h2)], db, o[m], 0, 0, 0);
-      }
+      for (int m = 0; m < MB; ++m)
+        o[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(tr.read(sk, m, j), db, o[m], 0, 0, 0);
     }
   });
 
   // with two key halves, half 1 hands its dQ^T to half 0 (same lane, same
-  // slots); the key loop ended on a barrier, so the tile buffers are free
+  // slots) through the tile buffers
   if constexpr (PK == 2) {
+    raw_barrier();  // every wave's copies were waited for, its reads are done
     float* s_o = (float*)s_t + qs * (MB * 16 * 64);
     if (kh == 1) {
 #pragma unroll
@@ -258,16 +314,21 @@ __global__ __launch_bounds__(PQ * PK * 64, 1) void attn_bwd_dq_kernel(AttnBwd p)
 }
 
 template <int HD, int PB, int PH>
-__global__ __launch_bounds__(PB * PH * 64, 1) void attn_bwd_dkv_kernel(AttnBwd p) {
+__global__ __launch_bounds__(PB * PH * 64, PH == 1 ? 2 : 1) void attn_bwd_dkv_kernel(AttnBwd p) {
   constexpr int PW = PB * PH;  // waves: key blocks x query parts
   constexpr int KS = HD / 16, MB = HD / 32, NCH = HD / 8, KT8 = 4 * HD;
-  constexpr int NKIND = 4;  // Q rows, dO rows, Q^T columns, dO^T columns
-  constexpr int NLD = NKIND * PH * KT8 / (PW * 64);
-  static_assert(NLD * PW * 64 == NKIND * PH * KT8, "loader coverage");
-  // two tile buffers (one barrier per iteration, as in the dQ kernel)
-  constexpr int NTILE = NKIND * PH * KT8, NMERGE = PH == 2 ? PB * 2 * MB * 16 * 64 * 4 / 16 : 0;
-  __shared__ f16x8 s_t[2 * NTILE > NMERGE ? 2 * NTILE : NMERGE];
-  __shared__ float s_ld[2][PH][2][32];  // log-sum-exp and D of the iteration's query blocks
+  constexpr int NB = 2;  // tile buffers: Q and dO rows of PH query blocks each
+  // The K and V rows, dK, dV, S and dP are 224 registers at hd = 128: with two
+  // workgroups per CU (PH = 1) each wave keeps its V rows in LDS instead.
+  constexpr bool VLDS = PH == 1 && HD == 128;
+  using Dma = TileDma<HD, PW, PH>;
+  constexpr int NTILE = 2 * PH * KT8, NMERGE = PH == 2 ? PB * 2 * MB * 16 * 64 * 4 / 16 : 0;
+  __shared__ f16x8 s_t[NB * NTILE > NMERGE ? NB * NTILE : NMERGE];
+  // log-sum-exp and D of the iteration's query blocks: [part][lse, D][64], the
+  // upper 32 of each a copy of the lower
+  __shared__ __align__(16) float s_ld[NB][PH][2][64];
+  static_assert(PW >= 2 * PH, "a wave copies one row of s_ld");
+  __shared__ f16x8 s_v[VLDS ? PB * KT8 : 1];
 
   const int tid = threadIdx.x, lane = tid & 63, h2 = lane >> 5, li = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -287,64 +348,54 @@ __global__ __launch_bounds__(PB * PH * 64, 1) void attn_bwd_dkv_kernel(AttnBwd p
   const int npairs = rep * nq;          // (head, query block) pairs
   const int niter = (npairs + PH - 1) / PH;
 
-  f16x8 kf[KS], vf[KS];
+  f16x8 kf[KS], vf[VLDS ? 1 : KS];
   if (active) {
     const size_t ko = ((size_t)z * p.Sp + ki) * HD + 8 * h2;
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
       kf[j] = *(const f16x8*)(p.k + ko + 16 * j);
-      vf[j] = *(const f16x8*)(p.v + ko + 16 * j);
+      if constexpr (!VLDS) vf[j] = *(const f16x8*)(p.v + ko + 16 * j);
     }
-  }
-
-  const size_t rq = (size_t)rep * p.Sp;
-  f16x8 reg[NLD];
-  float aux = 0.f;
-  auto pair_of = [&](int n, int hq, int& r, int& qb) {
-    const int pi = min(n * PH + hq, npairs - 1);
-    r = pi / nq;
-    qb = qstart + (pi - r * nq);
-  };
-  auto gload = [&](int n) {
+    if constexpr (VLDS) {  // this wave's own rows: its first dma_wait covers them
+      const i32x4 vrs = dma_rsrc(p.v + (size_t)z * p.Sp * HD);
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int x = i * PW * 64 + tid, tile = x / KT8, y = x % KT8;
-      const int kind = tile / PH;
-      int r, qb;
-      pair_of(n, tile % PH, r, qb);
-      if (kind < 2) {
-        const f16* base = kind == 0 ? p.q : p.dO;
-        const size_t row = ((size_t)b * p.H + g * rep + r) * p.Sp + qb * 32 + y / NCH;
-        reg[i] = *(const f16x8*)(base + row * HD + (y % NCH) * 8);
-      } else {
-        const f16* base = (kind == 2 ? p.qT : p.dOT) + (size_t)z * HD * rq;
-        reg[i] = *(const f16x8*)(base + (size_t)(y >> 2) * rq + (size_t)r * p.Sp + qb * 32 + (y & 3) * 8);
+      for (int n = 0; n < HD / 16; ++n) {
+        const int row = n * (64 / NCH) + lane / NCH;
+        dma_1k(lds_addr(s_v) + kbi * (HD * 64) + n * 1024,
+               (uint32_t)(row * HD + ((lane % NCH) ^ (swap23(row) % NCH)) * 8) * 2u, vrs,
+               (uint32_t)kb * (uint32_t)(HD * 64));
       }
     }
-    if (tid < PH * 2 * 32) {  // thread: (query half, lse or D, query)
-      const int hq = tid / 64, which = (tid >> 5) & 1, qq = tid & 31;
-      int r, qb;
-      pair_of(n, hq, r, qb);
-      const int qpos = qb * 32 + qq;
-      const size_t idx = ((size_t)b * p.H + g * rep + r) * p.Sp + qpos;
-      aux = qpos < p.S ? (which ? p.D[idx] : p.lse[idx]) : 0.f;
-    }
+  }
+  // LDS chunks of fragment j: base ^ 2j. The bases are made opaque in each
+  // iteration: hoisted out of the loop, the 16 addresses would spill.
+  const int qbase = swap23(li) * NCH + (h2 ^ (li % NCH)), vbase = li * NCH + (h2 ^ (swap23(li) % NCH));
+  auto vfrag = [&](int j, int vo) -> f16x8 {
+    if constexpr (VLDS)
+      return s_v[kbi * KT8 + (vo ^ (2 * j))];
+    else
+      return vf[j];
   };
-  auto lstore = [&](int buf) {
-    f16x8* st = s_t + buf * NTILE;
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int x = i * PW * 64 + tid, tile = x / KT8, y = x % KT8;
-      if (tile / PH < 2)
-        st[tile * KT8 + row_chunk<HD>(y / NCH, y % NCH)] = reg[i];
-      else
-        st[tile * KT8 + col_chunk(y >> 2, y & 3)] = reg[i];
-    }
-    if (tid < PH * 2 * 32) s_ld[buf][tid / 64][(tid >> 5) & 1][tid & 31] = aux;
+
+  // rows of the group's heads: row r*Sp + q of head g*rep + r, query q
+  const size_t grow = ((size_t)b * p.H + (size_t)g * rep) * p.Sp;
+  const Dma dma(p.q + grow * HD, p.dO + grow * HD, lds_addr(s_t), wave, lane);
+  const TrFrag<HD> tr(lane);
+  auto pair_row = [&](int n, int hq) {  // first row of the iteration's query block
+    const int pi = min(n * PH + hq, npairs - 1), r = pi / nq;
+    return r * p.Sp + (qstart + (pi - r * nq)) * 32;
+  };
+  // s_ld: waves beyond 2 * PH repeat the copy of wave % (2 * PH)
+  const int ldw = wave % (2 * PH);
+  const i32x4 ldrs = dma_rsrc((ldw & 1 ? p.D : p.lse) + grow);
+  const uint32_t ld_lds = lds_addr(&s_ld[0][0][0][0]) + ldw * 256;
+  auto issue = [&](int n, int buf) {
+    dma.issue(buf, [&](int part) { return pair_row(n, part); });
+    dma_256(ld_lds + buf * (uint32_t)sizeof(s_ld[0]), (uint32_t)li * 4u, ldrs,
+            (uint32_t)pair_row(n, ldw >> 1) * 4u);
   };
 
   const float sl2 = p.scale * HB_LOG2E;
-  const int qrow = swap23(li);
   f32x16 dk[MB], dv[MB];
 #pragma unroll
   for (int m = 0; m < MB; ++m) {
@@ -352,38 +403,55 @@ __global__ __launch_bounds__(PB * PH * 64, 1) void attn_bwd_dkv_kernel(AttnBwd p
     dv[m] = f32x16{};
   }
   auto body = [&](int n, int buf) {
-    if (!active || n * PH + qh >= npairs) return;  // wave-uniform
-    int r, qb;
-    pair_of(n, qh, r, qb);
+    const int pi = n * PH + qh;
+    if (!active || pi >= npairs) return;  // wave-uniform
+    const int qb = qstart + pi % nq;
     if (qb < kb) return;  // every query of the block precedes every key
-    const f16x8* st = s_t + buf * NTILE;
-    const f16x8* sq = st + (0 * PH + qh) * KT8;
-    const f16x8* sd = st + (1 * PH + qh) * KT8;
-    const f16x8* sqt = st + (2 * PH + qh) * KT8;
-    const f16x8* sdt = st + (3 * PH + qh) * KT8;
+    const f16x8* sq = s_t + buf * NTILE + qh * KT8;
+    const f16x8* sd = s_t + buf * NTILE + (PH + qh) * KT8;
     f32x16 s = {}, dp = {};
+    int qo = qbase, vo = vbase;
+    asm volatile("" : "+v"(qo), "+v"(vo));
+    constexpr int KH = KS / 2;  // fragments at a time: the registers are full
 #pragma unroll
-    for (int j = 0; j < KS; ++j) {
-      const int qo = qrow * NCH + ((2 * j + h2) ^ (li % NCH));
-      s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sq[qo], kf[j], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x16_f16(sd[qo], vf[j], dp, 0, 0, 0);
-    }
-    // rows are the queries qb*32 + swap23(slot), columns this lane's key ki;
-    // their log-sum-exp and D are read from LDS together, then masked
-    // entries get exp2(-inf) = 0 (a select on the argument, no branch)
-    float lq[16], dq[16];
+    for (int j0 = 0; j0 < KS; j0 += KH) {
+      f16x8 f[KH];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int qq = swap23(8 * (e >> 2) + 4 * h2 + (e & 3));
-      lq[e] = s_ld[buf][qh][0][qq];
-      dq[e] = s_ld[buf][qh][1][qq];
+      for (int j = 0; j < KH; ++j) f[j] = sq[qo ^ (2 * (j0 + j))];
+#pragma unroll
+      for (int j = 0; j < KH; ++j) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[j], kf[j0 + j], s, 0, 0, 0);
     }
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int qpos = qb * 32 + swap23(8 * (e >> 2) + 4 * h2 + (e & 3));
-      const float pe = exp2f((ki <= qpos && qpos < p.S) ? s[e] * sl2 - lq[e] : -INFINITY);
-      s[e] = pe;
-      dp[e] = pe * (dp[e] - dq[e]) * p.scale;
+    for (int j0 = 0; j0 < KS; j0 += KH) {
+      f16x8 f[KH];
+#pragma unroll
+      for (int j = 0; j < KH; ++j) f[j] = sd[qo ^ (2 * (j0 + j))];
+#pragma unroll
+      for (int j = 0; j < KH; ++j) dp = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[j], vfrag(j0 + j, vo), dp, 0, 0, 0);
+    }
+    // rows are the queries qb*32 + 16j + 8h2 + i (registers 8j + i), columns
+    // this lane's key ki
+#pragma unroll
+    for (int e = 0; e < 16; e += 4) {
+      const f32x4 l = *(const f32x4*)&s_ld[buf][qh][0][16 * (e >> 3) + 8 * h2 + (e & 7)];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[e + i] = s[e + i] * sl2 - l[i];
+    }
+    // masked entries only in the diagonal block and where the sequence ends
+    if (qb == kb || (qb + 1) * 32 > p.S) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int qpos = qb * 32 + 16 * (e >> 3) + 8 * h2 + (e & 7);
+        if (ki > qpos || qpos >= p.S) s[e] = -INFINITY;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] = __builtin_amdgcn_exp2f(s[e]);
+#pragma unroll
+    for (int e = 0; e < 16; e += 4) {
+      const f32x4 d = *(const f32x4*)&s_ld[buf][qh][1][16 * (e >> 3) + 8 * h2 + (e & 7)];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dp[e + i] = s[e + i] * (dp[e + i] - d[i]) * p.scale;
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -395,28 +463,24 @@ __global__ __launch_bounds__(PB * PH * 64, 1) void attn_bwd_dkv_kernel(AttnBwd p
       }
 #pragma unroll
       for (int m = 0; m < MB; ++m) {
-        const int c = col_chunk(m * 32 + li, 2 * j + h2);
-        dv[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sdt[c], pb, dv[m], 0, 0, 0);
-        dk[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sqt[c], db, dk[m], 0, 0, 0);
+        dv[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(tr.read(sd, m, j), pb, dv[m], 0, 0, 0);
+        dk[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(tr.read(sq, m, j), db, dk[m], 0, 0, 0);
       }
     }
   };
-  gload(0);
-  lstore(0);
-  if (niter > 1) gload(1);
-  lds_barrier();
+  // as the dQ kernel's key loop, one iteration ahead
+  issue(0, 0);
   for (int n = 0; n < niter; ++n) {
+    dma_wait<0>();
+    raw_barrier();
+    if (n + 1 < niter) issue(n + 1, (n + 1) & 1);
     body(n, n & 1);
-    if (n + 1 < niter) {
-      lstore((n + 1) & 1);  // that buffer was last read in iteration n - 1
-      if (n + 2 < niter) gload(n + 2);
-    }
-    lds_barrier();
   }
 
   // with two query halves, half 1 hands its dK^T and dV^T to half 0 of the
-  // same key block (the loop ended on a barrier: the tile buffers are free)
+  // same key block through the tile buffers
   if constexpr (PH == 2) {
+    raw_barrier();  // every wave's copies were waited for, its reads are done
     float* s_o = (float*)s_t + kbi * (2 * MB * 16 * 64);
     if (qh == 1) {
 #pragma unroll
@@ -459,31 +523,15 @@ __global__ __launch_bounds__(PB * PH * 64, 1) void attn_bwd_dkv_kernel(AttnBwd p
 }
 
 namespace {
-// Four query blocks (dQ) or four key blocks (dK/dV) per workgroup share each
-// staged tile once that still leaves two workgroups per CU (7B, one sequence
-// of 2048: forward + backward 136.1 -> 129.5 ms; 8 query blocks for dQ:
-// 125.0 -> 119.9 ms); otherwise two blocks, with the key or query range split
-// in halves.
-constexpr long HB_BWD_WIDE_MIN = 512;
+// Four query (dQ) or key (dK/dV) blocks per workgroup share each staged tile
+// once that gives every CU a workgroup; otherwise two blocks, with the key or
+// query range split in halves.
+constexpr long HB_BWD_WIDE_MIN = 256;
 template <int HD>
 void launch_bwd(const AttnBwd& p, hipStream_t st) {
   const int nb = (p.S + 31) / 32;
   const long hb = (long)p.H * p.B, zb = (long)p.KVH * p.B;
-  // dQ: 8 query blocks per workgroup (8 waves, hd = 128 only: one K, V and
-  // K^T tile set covers 512 threads' loads) while that still gives every CU
-  // one workgroup, else 4 with two workgroups per CU, else 2 with the key
-  // range split in halves. dK/dV: 4 key blocks, else 2 with the query range
-  // split (8 waves would need the K and V rows out of registers: the wave's
-  // dK, dV, K and V already fill 224 of its 256 registers)
-  bool dq8 = false;
-  if constexpr (HD == 128) {
-    if ((long)((nb + 7) / 8) * hb >= HB_BWD_WIDE_MIN / 2) {
-      hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, 8, 1>), dim3((nb + 7) / 8, p.H, p.B), dim3(512), 0, st, p);
-      dq8 = true;
-    }
-  }
-  if (dq8) {
-  } else if ((long)((nb + 3) / 4) * hb >= HB_BWD_WIDE_MIN)
+  if ((long)((nb + 3) / 4) * hb >= HB_BWD_WIDE_MIN)
     hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, 4, 1>), dim3((nb + 3) / 4, p.H, p.B), dim3(256), 0, st, p);
   else
     hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, 2, 2>), dim3((nb + 1) / 2, p.H, p.B), dim3(256), 0, st, p);

@@ -113,7 +113,7 @@ hipError_t cast_transpose(const float* src, int R, int C, float scale, f16* rm, 
 // HBM-bound: 4 V bytes read and 2 Vp written per position. The row stays in
 // registers (NV float4 per thread, V <= 2048 * NV), so it is read once with
 // 16-byte loads and each exponential is taken once: 2048 x 32000 from 230 us
-// (three passes of 4-byte loads) to CE_BWD_US. NV = 0: any V, in three passes.
+// (three passes of 4-byte loads) to 106. NV = 0: any V, in three passes.
 constexpr int CE_NT = 512;
 template <int NV>
 __global__ __launch_bounds__(CE_NT) void ce_backward_kernel(const float* __restrict__ logits,
@@ -373,7 +373,7 @@ size_t rmsnorm_backward_part_floats(int dim) { return (size_t)NORM_PARTS * dim; 
 // scheduling. Each wave finds the later occurrences 64 positions at a time
 // with a ballot (one token per lane, read straight from L2); the positions
 // walked one by one took 139 us at 2048 tokens of 4096 features, this
-// EMB_BWD_US.
+// 30 us.
 constexpr int EMB_MAX_DIM = 8192;  // 8 float4 per thread
 __global__ __launch_bounds__(256) void embed_bwd_kernel(const float* __restrict__ dx,
                                                         const uint32_t* __restrict__ tok, int T,

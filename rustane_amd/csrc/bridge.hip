@@ -193,7 +193,7 @@ struct TrainState {
   float* Drow = nullptr;  // [B][heads][Sp] rowsum(P * dP) of the attention backward
   f16 *d16 = nullptr, *d16T = nullptr, *dh = nullptr, *dhT = nullptr, *actT = nullptr;
   f16 *dqkv = nullptr, *dqkvT = nullptr, *dl = nullptr, *dlT = nullptr;
-  f16 *dA = nullptr, *dAT = nullptr, *qT = nullptr, *kT = nullptr, *vt = nullptr;
+  f16 *dA = nullptr, *vt = nullptr;
   // hb_train_forward left its activations for hb_train_backward (the
   // reference's ForwardResult.caches); any other training call clears it.
   bool kept = false;
@@ -2806,8 +2806,7 @@ int train_buffers(hb_model* m, int B, int S) {
   const size_t o_d16 = take(T * d * 2), o_d16T = take(d * Tp * 2), o_dh = take(T * 2 * h * 2),
                o_dhT = take(2 * h * Tp * 2), o_actT = take(actw * Tp * 2), o_dqkv = take(T * qkv * 2),
                o_dqkvT = take(qkv * Tp * 2), o_dl = take(T * Vp * 2), o_dlT = take(V * Tp * 2);
-  const size_t o_dA = take(qh * 2), o_dAT = take(qh * 2), o_qT = take(qh * 2), o_kT = take(kvh * 2),
-               o_vt = take(kvh * 2);
+  const size_t o_dA = take(qh * 2), o_vt = take(kvh * 2);
   hipStream_t st = m->ctx->stream();
   if (off > ts->abytes) {
     HIP_TRY(hipStreamSynchronize(st));
@@ -2836,8 +2835,7 @@ int train_buffers(hb_model* m, int B, int S) {
   ts->d16 = (f16*)(b + o_d16); ts->d16T = (f16*)(b + o_d16T); ts->dh = (f16*)(b + o_dh);
   ts->dhT = (f16*)(b + o_dhT); ts->actT = (f16*)(b + o_actT); ts->dqkv = (f16*)(b + o_dqkv);
   ts->dqkvT = (f16*)(b + o_dqkvT); ts->dl = (f16*)(b + o_dl); ts->dlT = (f16*)(b + o_dlT);
-  ts->dA = (f16*)(b + o_dA); ts->dAT = (f16*)(b + o_dAT); ts->qT = (f16*)(b + o_qT);
-  ts->kT = (f16*)(b + o_kT); ts->vt = (f16*)(b + o_vt);
+  ts->dA = (f16*)(b + o_dA); ts->vt = (f16*)(b + o_vt);
   HIP_TRY(fill_f16_zero((f16*)b, off / 2, st));
   ts->B = B;
   ts->S = S;
@@ -2890,28 +2888,20 @@ int train_forward(hb_model* m, int B, int S) {
 
 // Attention backward of one layer (kernels/sdpa_bwd.rs:46-161): the fused
 // kernels (attention_bwd.hip) recompute P from Q, K and the forward's
-// log-sum-exp, with the operands they read as MFMA A fragments transposed
-// first (K^T, and the rep = heads/kv_heads query heads of a group stacked as
-// [hd][rep*Sp] for Q^T and dO^T), and write dQ, dK, dV with RoPE^-1 into the
-// dQKV rows and their transpose.
+// log-sum-exp and write dQ, dK, dV with RoPE^-1 into the dQKV rows and their
+// transpose.
 int attention_backward(hb_model* m, const LayerAct& A, int B, int S) {
   const hb_model_config& c = m->cfg;
   TrainState* ts = m->train;
   hipStream_t st = m->ctx->stream();
-  const int Sp = (int)round64(S), T = B * S, Tp = (int)round64(T);
-  const int Z = B * c.kv_heads, rep = c.heads / c.kv_heads, Rq = rep * Sp, hd = c.hd;
-  const size_t khs = (size_t)Sp * hd, qzs = (size_t)Rq * hd;
-  HIP_TRY(transpose_f16(A.k, Sp, hd, hd, khs, ts->kT, Sp, khs, Z, st));
-  HIP_TRY(transpose_f16(A.q, Rq, hd, hd, qzs, ts->qT, Rq, qzs, Z, st));
-  HIP_TRY(transpose_f16(ts->dA, Rq, hd, hd, qzs, ts->dAT, Rq, qzs, Z, st));
+  const int Sp = (int)round64(S), T = B * S, Tp = (int)round64(T), hd = c.hd;
   AttnBwd p{};
-  p.q = A.q; p.dO = ts->dA; p.k = A.k; p.v = A.v; p.qT = ts->qT; p.dOT = ts->dAT; p.kT = ts->kT;
+  p.q = A.q; p.dO = ts->dA; p.k = A.k; p.v = A.v;
   p.lse = A.lse; p.D = ts->Drow;
   p.B = B; p.S = S; p.Sp = Sp; p.H = c.heads; p.KVH = c.kv_heads; p.hd = hd;
   p.scale = 1.0f / sqrtf((float)hd);
   p.dqkv = ts->dqkv; p.dqkvT = ts->dqkvT; p.ld = c.q_dim + 2 * c.kv_dim; p.tld = Tp;
   p.q_dim = c.q_dim; p.kv_dim = c.kv_dim; p.rope = m->rope; p.rope_ld = m->rope_len;
-  (void)T;
   HIP_TRY(attention_backward_fused(p, st));
   return HB_OK;
 }

@@ -10,6 +10,7 @@ typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 #define HB_DEV __device__ __forceinline__
 
@@ -54,6 +55,50 @@ HB_DEV void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// ---- direct global -> LDS copies ----
+// Buffer descriptor of 16-byte accesses anywhere in 4 GiB from base.
+HB_DEV i32x4 dma_rsrc(const void* base) {
+  const uint64_t a = (uint64_t)base;
+  return i32x4{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), -1, 0x00020000};
+}
+// One wave copies 64 x 16 bytes from global memory (per-lane byte offset voff,
+// wave-uniform soff, both from the buffer's base) straight into LDS at
+// lds + 16 * lane. No output register;
+// the copy is counted by vmcnt (dma_wait). The nop is the wait state between
+// the write of m0 and its use.
+HB_DEV void dma_1k(uint32_t lds, uint32_t voff, i32x4 rsrc, uint32_t soff) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc),
+      "s"(soff)
+      : "memory");
+}
+// The same with 64 x 4 bytes.
+HB_DEV void dma_256(uint32_t lds, uint32_t voff, i32x4 rsrc, uint32_t soff) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc),
+      "s"(soff)
+      : "memory");
+}
+// At most N of this wave's copies in flight; all its LDS reads done.
+template <int N>
+HB_DEV void dma_wait() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+// Barrier without the vmcnt drain of __syncthreads; no memory access moves
+// across it.
+HB_DEV void raw_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+}
+// LDS byte address of a __shared__ object, for dma_1k.
+template <class T>
+HB_DEV uint32_t lds_addr(T* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) T*)p;
 }
 
 // Wave-wide reductions (64 lanes). __shfl_xor lowers to an LDS permute

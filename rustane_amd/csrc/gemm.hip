@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_norm_kernel(const float* __
 // 4096 87 / 78 / 104 / 90 / 106 / 133; 22016 x 45 x 4096 69 / 55 / 46 / 43 / 31 /
 // 42. 192x128 and 128x128 workgroups run two to a CU.
 const GemmTile GEMM_TILES[6] = {{256, 256, 1.43f, 10.f}, {192, 256, 1.11f, 8.f},  {128, 256, 0.83f, 6.5f},
-                                {192, 128, 0.64f, 7.f},  {128, 128, 0.49f, 5.f},  {64, 128, 0.34f, 4.f}};
+                                {192, 128, 0.64f, 7.f},  {128, 128, 0.49f, 5.f},  {64, 128, 0.42f, 4.5f}};
 static constexpr int GEMM_CUS = 256;  // MI355X compute units
 
 GemmChoice gemm_tile(int N, int T, int K, int S, float* us) {

@@ -144,30 +144,6 @@ struct GemmPlan {
   }
 };
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-
-// One wave copies 64 x 16 bytes from global memory (per-lane byte offset voff,
-// wave-uniform soff) straight into LDS at lds + 16 * lane. No output register;
-// the copy is counted by vmcnt (dma_wait). The nop is the wait state between
-// the write of m0 and its use.
-HB_DEV void dma_1k(uint32_t lds, uint32_t voff, i32x4 rsrc, uint32_t soff) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc),
-      "s"(soff)
-      : "memory");
-}
-// At most N of this wave's copies in flight; all its LDS reads done.
-template <int N>
-HB_DEV void dma_wait() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
-}
-// Barrier without the vmcnt drain of __syncthreads.
-HB_DEV void raw_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 // The GEMM kernel: 8 waves (2 feature rows x 4 token columns), two per SIMD,
 // on v_mfma_f32_16x16x32_f16.
 //
@@ -225,10 +201,8 @@ __global__ __launch_bounds__(512, 1) void gemm_nt_kernel(const f16* __restrict__
   for (int i = 0; i < FM; ++i) wvo[i] = (uint32_t)(min(f_base + i * 64 + wave * 8 + lr, N - 1) * kw + lc * 8) * 2u;
 #pragma unroll
   for (int j = 0; j < 2 * TM; ++j) xvo[j] = (uint32_t)(min(t_base + j * 64 + wave * 8 + lr, T - 1) * K + lc * 8) * 2u;
-  const uint64_t wa = (uint64_t)W, xa = (uint64_t)X;
-  const i32x4 wrs = {(int)(uint32_t)wa, (int)(uint32_t)(wa >> 32), -1, 0x00020000};
-  const i32x4 xrs = {(int)(uint32_t)xa, (int)(uint32_t)(xa >> 32), -1, 0x00020000};
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) f16x8*)smem + wave * 1024;
+  const i32x4 wrs = dma_rsrc(W), xrs = dma_rsrc(X);
+  const uint32_t lds0 = lds_addr(smem) + wave * 1024;
   const int kt0 = blockIdx.y * kq;
   const int nk = min(kq, K / 64 - kt0);
   auto dma_w = [&](int i, int stage, int k) {

@@ -146,8 +146,6 @@ hipError_t attention_prefill(const AttnPrefill& p, hipStream_t st);
 struct AttnBwd {
   const f16 *q, *dO;      // [B][H][Sp][hd]
   const f16 *k, *v;       // [B][KVH][Sp][hd]
-  const f16 *qT, *dOT;    // per z = b*KVH + g: [hd][rep*Sp] (head r of the group at r*Sp)
-  const f16* kT;          // per z: [hd][Sp]
   const float* lse;       // [B][H][Sp], from attention_prefill
   float* D;               // [B][H][Sp] scratch, written by the dQ launch
   int B, S, Sp, H, KVH, hd;
