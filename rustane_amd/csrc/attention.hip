@@ -3,60 +3,59 @@
 //   A[s] = sum_t P[s,t] V[t].
 // The reference's additive -65504 underflows to exactly 0 after exp (every row
 // keeps its diagonal term), so masked keys are skipped instead of added.
+#include "attention_tiles.hpp"
 #include "internal.hpp"
 
 namespace hb {
 
-// ---- prefill: one workgroup of 4 waves per (64 queries, head, sequence) ---------
+// ---- prefill ------------------------------------------------------------------
 // S^T = K · Q^T on v_mfma_f32_32x32x16_f16 (rows = key slots, cols = queries):
 // lane l owns query l%32 and the key slots 8*(r/4) + 4*(l/32) + r%4 of the
 // 32-key block, so the online-softmax statistics of a query live in one lane
 // pair (l, l^32). Key slot R holds key swap23(R) (bits 2 and 3 of the slot
 // swapped), which makes the 8 score registers 8j..8j+7 of lane half h the
 // consecutive keys 16j+8h .. 16j+8h+7. O^T = V^T · P^T then reuses those
-// registers as the B operand, and the A operand (V^T row, the same 8 keys) is
-// one 16-byte read.
+// registers as the B operand; the A operand (a V column, the same 8 keys)
+// comes from the V rows through ds_read_b64_tr_b16 (TrFrag), so V is stored
+// in rows only: the QKV epilogue writes 8 bytes per store where V^T took four
+// 2-byte ones, and ragged lengths need no cleared columns.
 //
 // Wave w = qs + PQ*kh owns query block qs (of PQ) of the workgroup and the
-// key blocks kb with kb % PK == kh (PK = 2): iteration n loads key blocks
-// PK*n .. PK*n+PK-1 (K [32][hd] and V^T [hd][32] each) into LDS once, with
-// 16-byte, wave-contiguous loads issued one iteration ahead, and every block
-// is used by the PQ waves of its key half. Sharing a block between query
-// blocks halves the bytes loaded per MFMA — a wave loading its own K/V needs
-// ~128 B/clk per CU, four times what the L1-L2 path sustains — while splitting
-// the key range over PK waves keeps the chain of dependent key blocks at half
-// the row; the key halves merge through LDS at the end (the same rescaling an
-// online softmax applies between blocks). Fragments are read from
-// XOR-swizzled LDS without bank conflicts.
+// key blocks kb with kb % PK == kh: iteration n works on key blocks
+// PK*n .. PK*n+PK-1, whose K and V rows are copied straight into LDS NB - 1
+// iterations ahead (dma_1k: no registers, no LDS stores; one barrier per
+// iteration), and every block is used by the PQ waves of its key part. Sharing
+// a block between query blocks divides the bytes loaded per MFMA — a wave
+// loading its own K/V needs ~128 B/clk per CU, four times what the L1-L2 path
+// sustains — while splitting the key range over PK waves keeps the chain of
+// dependent key blocks at half the row; the key halves merge through LDS at
+// the end (the same rescaling an online softmax applies between blocks).
+// Fragments are read from XOR-swizzled LDS without bank conflicts. Workgroups
+// of 4 waves leave room for two or three on a CU, whose MFMAs and softmaxes
+// overlap.
 //
-// PQ = 4 (8 waves) for long or many sequences: each key block then serves 128
-// queries instead of 64, halving the L2 traffic per MFMA, once there are
-// enough groups of 4 query blocks to give every CU two workgroups; short
-// single sequences keep PQ = 2 (7B S = 512, B = 1: 256 workgroups). PQ = 8
-// with PK = 1 (8 waves, each over the whole key range of its query block, no
-// merge) once groups of 8 still give every CU one workgroup.
-
+// PK = 1 (each wave over the whole key range of its query block, no merge)
+// once groups of 8 query blocks would still give every CU one workgroup, PK = 2
+// below: the split fixes the order of a query's sums, PQ does not.
 
 // SPLIT: Q, K, V and the probabilities in two-term fp16 form (common.hpp):
 // each score and output product runs hi*hi + hi*lo + lo*hi MFMAs (the lo*lo
 // term is below fp32 rounding of the sum), and the output rows are split rows.
 template <int HD, bool SPLIT, int PQ, int PK>
-__global__ __launch_bounds__(PQ * PK * 64, (SPLIT || PK == 1) ? 1 : 2) void attn_prefill_kernel(AttnPrefill p) {
+__global__ __launch_bounds__(PQ * PK * 64, SPLIT ? 1 : 2) void attn_prefill_kernel(AttnPrefill p) {
   constexpr int PW = PQ * PK;          // waves
   constexpr int KS = HD / 16;          // k-steps over head dim
   constexpr int MB = HD / 32;          // 32-row blocks of O^T
-  constexpr int NCH = HD / 8;          // 16-byte chunks per K row
-  constexpr int KT8 = 4 * HD;          // 16-byte chunks per K tile (= per V^T tile)
-  constexpr int NKIND = SPLIT ? 4 : 2;  // tile kinds: K, V^T (then their low parts)
-  constexpr int NLD = NKIND * PK * KT8 / (PW * 64);  // 16-byte loads per thread per iteration
-  static_assert(NLD * PW * 64 == NKIND * PK * KT8, "loader coverage");
-  // K tiles (block kh: row r, chunk c at kh*KT8 + r*NCH + (c ^ (swap23(r) % NCH))), then
-  // V^T tiles (block kh: row e, chunk c at (PK+kh)*KT8 + e*4 + (c ^ ((e >> 2) & 3))),
-  // then (SPLIT) the same two for the low parts; after the loop the region
-  // holds the key-half-1 waves' O for the merge
+  constexpr int NCH = HD / 8;          // 16-byte chunks per row
+  constexpr int KT8 = 4 * HD;          // 16-byte chunks per tile
+  constexpr int NKIND = SPLIT ? 4 : 2;  // tile kinds: K, V (then their low parts)
+  constexpr int NB = PK == 1 && !SPLIT ? 3 : 2;  // tile buffers
+  using Dma = TileDma<HD, PW, NKIND, PK>;
+  // a buffer's tiles are (kind, key part); after the loop the region holds the
+  // key-half-1 waves' O for the merge
   constexpr int NTILE = NKIND * PK * KT8, NMERGE = PK == 2 ? PQ * MB * 16 * 64 * 4 / 16 : 0;
-  __shared__ f16x8 s_kv[NTILE > NMERGE ? NTILE : NMERGE];
-  __shared__ float s_ml[PQ][2][64];
+  __shared__ f16x8 s_kv[NB * NTILE > NMERGE ? NB * NTILE : NMERGE];
+  __shared__ float s_ml[PK == 2 ? PQ : 1][2][64];
   const int tid = threadIdx.x, lane = tid & 63, h2 = lane >> 5, li = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
   const int qs = wave % PQ, kh = wave / PQ;
@@ -70,14 +69,15 @@ __global__ __launch_bounds__(PQ * PK * 64, (SPLIT || PK == 1) ? 1 : 2) void attn
   const int nwg = gridDim.x * gridDim.y * gridDim.z;
   const int wg = xcd_remap(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), nwg);
   const int gx = wg % gridDim.x, hy = (wg / gridDim.x) % gridDim.y, bz = wg / (gridDim.x * gridDim.y);
-  const int gr = ngr - 1 - gx;  // heaviest groups first within a head
-  // group gr holds the query blocks gr, gr + ngr, gr + 2 ngr, ...: every
-  // group spans the sequence, so the groups' causal work is nearly equal
-  // (contiguous groups left most CUs idle behind the last one); the
-  // arithmetic of a query block does not depend on its group
-  const int qb = gr + ngr * qs;  // >= nqb: this wave has no queries
+  // Group gr holds the query blocks PQ*gr .. PQ*gr + PQ-1, so its waves walk
+  // nearly the same keys; heaviest groups first within a head, with more
+  // workgroups than fit at a time filling up behind them. (Groups strided over
+  // the sequence have equal work, but their light waves idle: 7B, two of
+  // 2048, QKV + attention 438 against 430 us; 5B, one of 2048, 125 against 119.)
+  const int gr = ngr - 1 - gx;
+  const int qb = gr * PQ + qs;  // >= nqb: this wave has no queries
   const bool active = qb < nqb;
-  const int nkb = gr + ngr * min(PQ - 1, (nqb - 1 - gr) / ngr) + 1;  // key blocks the group needs
+  const int nkb = min(nqb, gr * PQ + PQ);  // key blocks the group needs
   const int h = hy, b = bz;
   const int kvh = h / (p.H / p.KVH);
   const int q0 = qb * 32;
@@ -94,64 +94,17 @@ __global__ __launch_bounds__(PQ * PK * 64, (SPLIT || PK == 1) ? 1 : 2) void attn
     }
   }
 
-  const size_t koff = b * p.k_bstride + kvh * p.k_hstride;
-  const size_t voff = ((size_t)b * p.KVH + kvh) * HD * p.vt_ld;
+  const size_t koff = b * p.k_bstride + kvh * p.k_hstride, voff = b * p.v_bstride + kvh * p.v_hstride;
+  typename Dma::Bases bases;
+  bases.p[0] = p.k + koff;
+  bases.p[1] = p.v + voff;
+  if constexpr (SPLIT) {
+    bases.p[2] = p.k_lo + koff;
+    bases.p[3] = p.v_lo + voff;
+  }
+  const Dma dma(bases, lds_addr(s_kv), wave, lane);
+  const TrFrag<HD> tr(lane);
   const float sl2 = p.scale * HB_LOG2E;
-
-  // thread tid, load i covers 16-byte chunk x = i*NT + tid (NT = PW*64) of the
-  // iteration's NKIND*PK tiles (K blocks, then V^T blocks, then their low
-  // parts). NT and KT8 are powers of two, so x's tile is a constant of i, or
-  // of i and the wave when NT > KT8: written that way, the branches on the
-  // tile kind below are uniform (from tid alone the compiler made them
-  // divergent, with a wait in each).
-  constexpr int NT = PW * 64;
-  auto tile_of = [&](int i) {
-    if constexpr (NT <= KT8)
-      return (i * NT) / KT8;
-    else
-      return i * (NT / KT8) + (wave * 64) / KT8;
-  };
-  auto y_of = [&](int i) {
-    if constexpr (NT <= KT8)
-      return (i * NT) % KT8 + tid;
-    else
-      return tid % KT8;
-  };
-  static_assert(NT <= KT8 ? KT8 % NT == 0 : NT % KT8 == 0, "tiles and threads nest");
-  f16x8 kvreg[NLD];
-  auto gload = [&](int n) {
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int tile = tile_of(i), y = y_of(i);
-      const int kind = tile / PK;  // 0 K, 1 V^T, 2 K low, 3 V^T low
-      const int kb = min(n * PK + (tile % PK), nkb - 1);
-      if ((kind & 1) == 0) {
-        const f16* kbase = (kind ? p.k_lo : p.k) + koff;
-        kvreg[i] = *(const f16x8*)(kbase + ((size_t)kb * 32 + y / NCH) * HD + (y % NCH) * 8);
-      } else {
-        const f16* vbase = (kind > 1 ? p.vt_lo : p.vt) + voff;
-        const int e = y >> 2, c = y & 3;
-        kvreg[i] = *(const f16x8*)(vbase + (size_t)e * p.vt_ld + kb * 32 + c * 8);
-      }
-    }
-  };
-  auto lstore = [&]() {
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int tile = tile_of(i), y = y_of(i);
-      if (((tile / PK) & 1) == 0) {
-        const int r = y / NCH, c = y % NCH;
-        s_kv[tile * KT8 + r * NCH + (c ^ (swap23(r) % NCH))] = kvreg[i];
-      } else {
-        const int e = y >> 2, c = y & 3;
-        s_kv[tile * KT8 + e * 4 + (c ^ ((e >> 2) & 3))] = kvreg[i];
-      }
-    }
-  };
-  const f16x8* sk = s_kv + kh * KT8;
-  const f16x8* sv = s_kv + (PK + kh) * KT8;
-  const f16x8* skl = s_kv + (2 * PK + kh) * KT8;  // SPLIT only
-  const f16x8* svl = s_kv + (3 * PK + kh) * KT8;
 
   f32x16 o[MB];
 #pragma unroll
@@ -160,14 +113,29 @@ __global__ __launch_bounds__(PQ * PK * 64, (SPLIT || PK == 1) ? 1 : 2) void attn
 
   const int krow = swap23(li);  // key held in this lane's slot
   const int niter = (nkb + PK - 1) / PK;
-  gload(0);
-  for (int n = 0; n < niter; ++n) {
-    lds_barrier();  // every wave is done with the previous iteration's tiles
-    lstore();
-    lds_barrier();  // the tiles are in LDS
-    if (n + 1 < niter) gload(n + 1);
+  auto issue = [&](int n, int buf) {
+    dma.issue(buf, [&](int part) { return min(n * PK + part, nkb - 1) * 32; });
+  };
+  issue(0, 0);
+  if (NB == 3 && niter > 1) issue(1, 1);
+  settle(qf);
+  if constexpr (SPLIT) settle(ql);
+  int buf = 0;
+  for (int n = 0; n < niter; ++n, buf = buf == NB - 1 ? 0 : buf + 1) {
+    // The barrier follows every wave's wait for its own copies of iteration n
+    // and its last read of n - 1, whose buffer the new copies go into.
+    if (NB == 3 && n + 1 < niter)
+      dma_wait<Dma::NI>();
+    else
+      dma_wait<0>();
+    raw_barrier();
+    if (n + NB - 1 < niter) issue(n + NB - 1, buf == 0 ? NB - 1 : buf - 1);
     const int kb = n * PK + kh;
     if (!active || kb > qb) continue;  // wave-uniform
+    const f16x8* sk = s_kv + buf * NTILE + kh * KT8;
+    const f16x8* sv = sk + PK * KT8;
+    const f16x8* skl = sk + 2 * PK * KT8;  // SPLIT only
+    const f16x8* svl = sk + 3 * PK * KT8;
 
     // all of the block's K fragments are read before the score MFMAs, so
     // the LDS reads overlap instead of each waiting in front of its MFMA
@@ -227,6 +195,17 @@ __global__ __launch_bounds__(PQ * PK * 64, (SPLIT || PK == 1) ? 1 : 2) void attn
       lrun += e;  // this lane's keys; the lane pair is summed after the loop
     }
 
+    // V rows past the sequence may hold anything; they meet probability 0 and
+    // must not be NaN. Only this wave reads the last key block's tile (every
+    // other query block of the group comes before it), so it clears them there.
+    if (kb * 32 + 32 > p.S) {
+      const int past = p.S - kb * 32;
+      for (int x = lane; x < KT8; x += 64)
+        if (x / NCH >= past) {
+          s_kv[buf * NTILE + (PK + kh) * KT8 + x] = f16x8{};
+          if constexpr (SPLIT) s_kv[buf * NTILE + (3 * PK + kh) * KT8 + x] = f16x8{};
+        }
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       f16x8 pb, pl;
@@ -238,13 +217,11 @@ __global__ __launch_bounds__(PQ * PK * 64, (SPLIT || PK == 1) ? 1 : 2) void attn
       }
 #pragma unroll
       for (int m = 0; m < MB; ++m) {
-        const int e = m * 32 + li;
-        const int vo = e * 4 + ((2 * j + h2) ^ ((e >> 2) & 3));
-        const f16x8 va = sv[vo];
+        const f16x8 va = tr.read(sv, m, j);
         o[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb, o[m], 0, 0, 0);
         if constexpr (SPLIT) {
           o[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pl, o[m], 0, 0, 0);
-          o[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(svl[vo], pb, o[m], 0, 0, 0);
+          o[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(tr.read(svl, m, j), pb, o[m], 0, 0, 0);
         }
       }
     }
@@ -258,7 +235,7 @@ __global__ __launch_bounds__(PQ * PK * 64, (SPLIT || PK == 1) ? 1 : 2) void attn
   float M = mrun, L = lrun;
   if constexpr (PK == 2) {
     float* s_o = (float*)s_kv + qs * (MB * 16 * 64);  // [MB*16][64] per query block
-    lds_barrier();  // every wave is done with the tiles
+    raw_barrier();  // every wave's copies were waited for, its reads are done
     if (kh == 1) {
 #pragma unroll
       for (int m = 0; m < MB; ++m)
@@ -322,14 +299,9 @@ hipError_t launch_prefill(const AttnPrefill& p, hipStream_t st) {
 }  // namespace
 
 hipError_t attention_prefill(const AttnPrefill& p, hipStream_t st) {
-  if (p.q_lo != nullptr && (!p.k_lo || !p.vt_lo)) return hipErrorInvalidValue;
-  // PQ = 8 (one workgroup per CU) or 4 (two) when the grid still fills the
-  // GPU (measured on the 7B shape: seq 2048 forward at B = 1 33.2 ms with
-  // PQ = 2, 32.75 with 4, 31.5 -> 31.2 with 8; seq 512 at B = 8 55.7 -> 55.2)
+  if (p.q_lo != nullptr && (!p.k_lo || !p.v_lo)) return hipErrorInvalidValue;
   const int nqb = (p.S + 31) / 32;
-  const long hb = (long)p.H * p.B;
-  if ((long)((nqb + 7) / 8) * hb >= 256) return launch_prefill<8, 1>(p, st);
-  if ((long)((nqb + 3) / 4) * hb >= 512) return launch_prefill<4, 2>(p, st);
+  if ((long)((nqb + 7) / 8) * p.H * p.B >= 256) return launch_prefill<4, 1>(p, st);
   return launch_prefill<2, 2>(p, st);
 }
 

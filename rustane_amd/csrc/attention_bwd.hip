@@ -34,6 +34,7 @@
 // the group (the GQA sum over heads is the loop), dV^T += dO^T P and
 // dK^T += Q^T dS; with two query halves (PB = 2) the halves add their
 // partials through LDS.
+#include "attention_tiles.hpp"
 #include "internal.hpp"
 
 namespace hb {
@@ -68,74 +69,6 @@ HB_DEV void store_grad4(const AttnBwd& p, int b, int s, int col, int f0, f32x4 v
   p.dqkvT[(size_t)(col + 3) * p.tld + tok] = h.w;
 }
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
-// Transposed A fragments of a row tile. ds_read_b64_tr_b16: in each group of
-// 16 lanes, lane s supplies 4 halves of its own address and lane i receives,
-// as element e, half i%4 of lane 4e + i/4. With lane s at row base + s/4,
-// features F + 4(s%4)..+3, lane i gets feature F + i of rows base..base+3.
-// The fragment (m, j) of lane (h2, li) is feature m*32 + li of rows 16j + 8h2
-// .. +7: two reads. The tile's chunk swizzle enters through the two lane
-// bases (m even, odd); everything else is an immediate offset.
-template <int HD>
-struct TrFrag {
-  static constexpr int NCH = HD / 8;
-  int base[2];
-  HB_DEV explicit TrFrag(int lane) {
-    const int s = lane & 15, g = lane >> 4, h2 = lane >> 5;
-#pragma unroll
-    for (int mm = 0; mm < 2; ++mm) {
-      const int c = mm * 4 + 2 * (g & 1) + ((s & 3) >> 1), x = (4 * h2 + (s >> 2)) % NCH;
-      base[mm] = ((8 * h2 + (s >> 2)) * NCH + (c ^ x)) * 8 + 4 * (s & 1);
-    }
-  }
-  HB_DEV f16x8 read(const f16x8* tile, int m, int j) const {
-    const f16* t = (const f16*)tile + base[m & 1];
-    s16x4 v[2];
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int off = (16 * j + 4 * hh) * NCH * 8 + (NCH == 16 ? ((hh ^ (m >> 1)) & 1) * 64 : 0);
-      v[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (__attribute__((address_space(3))) s16x4*)(__attribute__((address_space(3))) void*)(t + off));
-    }
-    const auto w = __builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7);
-    return __builtin_bit_cast(f16x8, w);
-  }
-};
-
-// Copies of one iteration's tiles by PW waves: tile t = kind * PARTS + part is
-// 32 rows of HD halves at base[kind] + row0(part) * HD, NI instructions of
-// 1 KB per wave.
-template <int HD, int PW, int PARTS>
-struct TileDma {
-  static constexpr int NCH = HD / 8, IPT = HD / 16;  // instructions per tile
-  static constexpr int NI = 2 * PARTS * IPT / PW;
-  static constexpr uint32_t BYTES = 2 * PARTS * HD * 64;
-  static_assert(IPT % PW == 0, "an instruction slot belongs to one tile");
-  uint32_t voff[IPT / PW];
-  uint32_t lds;
-  i32x4 rs[2];
-  HB_DEV TileDma(const f16* b0, const f16* b1, uint32_t lds0, int wave, int lane) : lds(lds0 + wave * 1024) {
-    rs[0] = dma_rsrc(b0);
-    rs[1] = dma_rsrc(b1);
-#pragma unroll
-    for (int u = 0; u < IPT / PW; ++u) {
-      const int row = (wave + PW * u) * (64 / NCH) + lane / NCH;
-      voff[u] = (uint32_t)(row * HD + ((lane % NCH) ^ (swap23(row) % NCH)) * 8) * 2u;
-    }
-  }
-  // row0: (kind, part) -> first row, wave-uniform
-  template <class F>
-  HB_DEV void issue(int buf, F&& row0) const {
-#pragma unroll
-    for (int u = 0; u < NI; ++u) {
-      const int tile = u * PW / IPT, kind = tile / PARTS, part = tile % PARTS;
-      dma_1k(lds + buf * BYTES + u * PW * 1024, voff[u % (IPT / PW)], rs[kind],
-             (uint32_t)row0(part) * (uint32_t)(HD * 2));
-    }
-  }
-};
-
 }  // namespace
 
 template <int HD, int PQ, int PK>
@@ -143,7 +76,7 @@ __global__ __launch_bounds__(PQ * PK * 64, 2) void attn_bwd_dq_kernel(AttnBwd p)
   constexpr int PW = PQ * PK;  // waves: query blocks x key parts
   constexpr int KS = HD / 16, MB = HD / 32, NCH = HD / 8, KT8 = 4 * HD;
   constexpr int NB = PK == 1 ? 3 : 2;  // tile buffers: K and V rows of PK key blocks each
-  using Dma = TileDma<HD, PW, PK>;
+  using Dma = TileDma<HD, PW, 2, PK>;
   constexpr int NTILE = 2 * PK * KT8, NMERGE = PK == 2 ? PQ * MB * 16 * 64 * 4 / 16 : 0;
   __shared__ f16x8 s_t[NB * NTILE > NMERGE ? NB * NTILE : NMERGE];
   __shared__ float s_d[PQ][64];
@@ -175,8 +108,11 @@ __global__ __launch_bounds__(PQ * PK * 64, 2) void attn_bwd_dq_kernel(AttnBwd p)
     }
     if (qi < p.S) L2 = p.lse[qrow + qi];
   }
+  settle(qf);
+  settle(df);
+  asm volatile("" : "+v"(L2));
 
-  const Dma dma(p.k + (size_t)z * p.Sp * HD, p.v + (size_t)z * p.Sp * HD, lds_addr(s_t), wave, lane);
+  const Dma dma({p.k + (size_t)z * p.Sp * HD, p.v + (size_t)z * p.Sp * HD}, lds_addr(s_t), wave, lane);
   const TrFrag<HD> tr(lane);
   const float sl2 = p.scale * HB_LOG2E;
   const int krow = swap23(li);
@@ -321,7 +257,7 @@ __global__ __launch_bounds__(PB * PH * 64, PH == 1 ? 2 : 1) void attn_bwd_dkv_ke
   // The K and V rows, dK, dV, S and dP are 224 registers at hd = 128: with two
   // workgroups per CU (PH = 1) each wave keeps its V rows in LDS instead.
   constexpr bool VLDS = PH == 1 && HD == 128;
-  using Dma = TileDma<HD, PW, PH>;
+  using Dma = TileDma<HD, PW, 2, PH>;
   constexpr int NTILE = 2 * PH * KT8, NMERGE = PH == 2 ? PB * 2 * MB * 16 * 64 * 4 / 16 : 0;
   __shared__ f16x8 s_t[NB * NTILE > NMERGE ? NB * NTILE : NMERGE];
   // log-sum-exp and D of the iteration's query blocks: [part][lse, D][64], the
@@ -379,7 +315,7 @@ __global__ __launch_bounds__(PB * PH * 64, PH == 1 ? 2 : 1) void attn_bwd_dkv_ke
 
   // rows of the group's heads: row r*Sp + q of head g*rep + r, query q
   const size_t grow = ((size_t)b * p.H + (size_t)g * rep) * p.Sp;
-  const Dma dma(p.q + grow * HD, p.dO + grow * HD, lds_addr(s_t), wave, lane);
+  const Dma dma({p.q + grow * HD, p.dO + grow * HD}, lds_addr(s_t), wave, lane);
   const TrFrag<HD> tr(lane);
   auto pair_row = [&](int n, int hq) {  // first row of the iteration's query block
     const int pi = min(n * PH + hq, npairs - 1), r = pi / nq;
@@ -470,6 +406,8 @@ __global__ __launch_bounds__(PB * PH * 64, PH == 1 ? 2 : 1) void attn_bwd_dkv_ke
   };
   // as the dQ kernel's key loop, one iteration ahead
   issue(0, 0);
+  settle(kf);
+  settle(vf);
   for (int n = 0; n < niter; ++n) {
     dma_wait<0>();
     raw_barrier();

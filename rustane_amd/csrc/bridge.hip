@@ -86,18 +86,18 @@ struct LayerW {
   f16 *t_wqkv = nullptr, *t_wo = nullptr, *t_w13 = nullptr, *t_w2 = nullptr;
 };
 
-// Prefill activations. Q/K/V^T rows are padded per sequence to S_pad (multiple
+// Prefill activations. Q/K/V rows are padded per sequence to S_pad (multiple
 // of 32) for the attention kernel.
 struct Workspace {
   long cap_T = 0, cap_Tpad = 0;
   void* base = nullptr;
   float *x = nullptr, *x2 = nullptr, *logits = nullptr, *loss = nullptr, *mean = nullptr;
-  f16 *xn = nullptr, *q = nullptr, *k = nullptr, *vt = nullptr, *attn = nullptr, *gate = nullptr;
+  f16 *xn = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *attn = nullptr, *gate = nullptr;
   uint32_t *tok = nullptr, *tgt = nullptr;
   // split-operand layers (hb_model::precise_layers): xn, attn and gate have
-  // room for split rows [T, 2K], and Q, K, V^T have low parts
+  // room for split rows [T, 2K], and Q, K, V have low parts
   bool split = false;
-  f16 *q_lo = nullptr, *k_lo = nullptr, *vt_lo = nullptr;
+  f16 *q_lo = nullptr, *k_lo = nullptr, *v_lo = nullptr;
 };
 
 }  // namespace
@@ -193,7 +193,7 @@ struct TrainState {
   float* Drow = nullptr;  // [B][heads][Sp] rowsum(P * dP) of the attention backward
   f16 *d16 = nullptr, *d16T = nullptr, *dh = nullptr, *dhT = nullptr, *actT = nullptr;
   f16 *dqkv = nullptr, *dqkvT = nullptr, *dl = nullptr, *dlT = nullptr;
-  f16 *dA = nullptr, *vt = nullptr;
+  f16* dA = nullptr;
   // hb_train_forward left its activations for hb_train_backward (the
   // reference's ForwardResult.caches); any other training call clears it.
   bool kept = false;
@@ -359,10 +359,10 @@ int ensure_workspace(hb_model* m, long T, long Tpad, bool need_split = false) {
   const size_t o_xn = take(sf * T * c.dim * 2), o_attn = take(sf * T * c.q_dim * 2);
   const size_t o_gate = take(sf * (size_t)T * c.hidden * 2);
   const size_t o_q = take(Tpad * c.q_dim * 2), o_k = take(Tpad * c.kv_dim * 2);
-  const size_t o_vt = take(Tpad * c.kv_dim * 2);
+  const size_t o_v = take(Tpad * c.kv_dim * 2);
   const size_t o_tok = take(T * 4), o_tgt = take(T * 4);
   const size_t o_qlo = split ? take(Tpad * c.q_dim * 2) : 0, o_klo = split ? take(Tpad * c.kv_dim * 2) : 0;
-  const size_t o_vtlo = split ? take(Tpad * c.kv_dim * 2) : 0;
+  const size_t o_vlo = split ? take(Tpad * c.kv_dim * 2) : 0;
   char* base = nullptr;
   HIP_TRY(hipMalloc(&base, off));
   w.base = base;
@@ -372,7 +372,7 @@ int ensure_workspace(hb_model* m, long T, long Tpad, bool need_split = false) {
   if (split) {
     w.q_lo = (f16*)(base + o_qlo);
     w.k_lo = (f16*)(base + o_klo);
-    w.vt_lo = (f16*)(base + o_vtlo);
+    w.v_lo = (f16*)(base + o_vlo);
   }
   w.x = (float*)(base + o_x);
   w.x2 = (float*)(base + o_x2);
@@ -384,19 +384,19 @@ int ensure_workspace(hb_model* m, long T, long Tpad, bool need_split = false) {
   w.gate = (f16*)(base + o_gate);
   w.q = (f16*)(base + o_q);
   w.k = (f16*)(base + o_k);
-  w.vt = (f16*)(base + o_vt);
+  w.v = (f16*)(base + o_v);
   w.tok = (uint32_t*)(base + o_tok);
   w.tgt = (uint32_t*)(base + o_tgt);
-  // Padding rows/columns of Q, K and V^T are read (and masked) by attention:
+  // Padding rows of Q, K and V are read (and masked) by attention:
   // keep them finite.
   hipStream_t st = m->ctx->stream();
   HIP_TRY(fill_f16_zero(w.q, (size_t)Tpad * c.q_dim, st));
   HIP_TRY(fill_f16_zero(w.k, (size_t)Tpad * c.kv_dim, st));
-  HIP_TRY(fill_f16_zero(w.vt, (size_t)Tpad * c.kv_dim, st));
+  HIP_TRY(fill_f16_zero(w.v, (size_t)Tpad * c.kv_dim, st));
   if (split) {
     HIP_TRY(fill_f16_zero(w.q_lo, (size_t)Tpad * c.q_dim, st));
     HIP_TRY(fill_f16_zero(w.k_lo, (size_t)Tpad * c.kv_dim, st));
-    HIP_TRY(fill_f16_zero(w.vt_lo, (size_t)Tpad * c.kv_dim, st));
+    HIP_TRY(fill_f16_zero(w.v_lo, (size_t)Tpad * c.kv_dim, st));
   }
   return HB_OK;
 }
@@ -503,13 +503,11 @@ int ensure_decode_weights(hb_model* m) {
 struct KVTarget {
   f16* k;
   size_t k_bstride, k_hstride;
-  f16* v;  // nullable
+  f16* v;
   size_t v_bstride, v_hstride;
-  // low parts for split-operand layers, same strides (v_lo nullable)
+  // low parts for split-operand layers, same strides
   f16 *k_lo = nullptr, *v_lo = nullptr;
 };
-
-int zero_vt_pad(hb_model* m, f16* vt, int B, int S, hipStream_t st);
 
 // xn_ready: w.xn already holds RMSNorm1(x) (the previous layer's W2 produced
 // it). next_gamma != NULL: also leave RMSNorm(x_out, next_gamma) in w.xn for
@@ -588,18 +586,13 @@ int run_layer(hb_model* m, int l, int B, int S, const KVTarget& kv, float* qkv_t
   e.v = kv.v;
   e.v_bstride = kv.v_bstride;
   e.v_hstride = kv.v_hstride;
-  e.vt = w.vt;
-  e.vt_ld = Sp;
   e.tap = qkv_tap;
   if (sp) {
     e.q_lo = w.q_lo;
     e.k_lo = kv.k_lo;
     e.v_lo = kv.v_lo;
-    e.vt_lo = w.vt_lo;
   }
   HIP_TRY(gemm_qkv(L.wqkv, w.xn, c.q_dim + 2 * c.kv_dim, T, f * c.dim, e, st, c.dim));
-  TRY(zero_vt_pad(m, w.vt, B, S, st));
-  if (sp) TRY(zero_vt_pad(m, w.vt_lo, B, S, st));
   HB_MARK(tm, ST_QKV);
   AttnPrefill a{};
   a.q = w.q;
@@ -607,8 +600,9 @@ int run_layer(hb_model* m, int l, int B, int S, const KVTarget& kv, float* qkv_t
   a.k = kv.k;
   a.k_bstride = kv.k_bstride;
   a.k_hstride = kv.k_hstride;
-  a.vt = w.vt;
-  a.vt_ld = Sp;
+  a.v = kv.v;
+  a.v_bstride = kv.v_bstride;
+  a.v_hstride = kv.v_hstride;
   a.out = w.attn;
   a.B = B;
   a.S = S;
@@ -619,7 +613,7 @@ int run_layer(hb_model* m, int l, int B, int S, const KVTarget& kv, float* qkv_t
   if (sp) {
     a.q_lo = w.q_lo;
     a.k_lo = kv.k_lo;
-    a.vt_lo = w.vt_lo;
+    a.v_lo = kv.v_lo;
   }
   HIP_TRY(attention_prefill(a, st));
   HB_MARK(tm, ST_ATTN);
@@ -653,30 +647,15 @@ KVTarget scratch_kv(hb_model* m, int B, int S) {
   t.k = m->ws.k;
   t.k_hstride = (size_t)Sp * c.hd;
   t.k_bstride = (size_t)c.kv_heads * t.k_hstride;
-  t.v = nullptr;
+  t.v = m->ws.v;
+  t.v_bstride = t.k_bstride;
+  t.v_hstride = t.k_hstride;
   t.k_lo = m->ws.k_lo;
+  t.v_lo = m->ws.v_lo;
   (void)B;
   return t;
 }
 
-}  // namespace
-
-// Zero the V^T columns [S, S_pad) so masked (p = 0) keys never meet a NaN.
-__global__ void zero_vt_pad_kernel(f16* vt, int rows, int ld, int S) {
-  const int r = blockIdx.x * 4 + (threadIdx.x >> 5);
-  const int c = S + (threadIdx.x & 31);
-  if (r < rows && c < ld) vt[(size_t)r * ld + c] = (f16)0.f;
-}
-
-namespace {
-int zero_vt_pad(hb_model* m, f16* vt, int B, int S, hipStream_t st) {
-  const int Sp = S_pad_of(S);
-  if (Sp == S) return HB_OK;
-  const int rows = B * m->cfg.kv_heads * m->cfg.hd;
-  hipLaunchKernelGGL(zero_vt_pad_kernel, dim3((rows + 3) / 4), dim3(128), 0, st, vt, rows, Sp, S);
-  HIP_TRY(hipGetLastError());
-  return HB_OK;
-}
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -2202,13 +2181,12 @@ extern "C" int hb_op_sdpa_fwd(hb_model* m, int layer, const void* xnorm, int B, 
   e.q_dim = c.q_dim; e.kv_dim = c.kv_dim; e.hd = c.hd; e.S = S; e.heads = c.heads;
   e.kv_heads = c.kv_heads; e.rope = m->rope; e.rope_ld = m->rope_len; e.d_pos = nullptr;
   e.q = w.q; e.q_rows = Sp;
-  e.k = kv.k; e.k_bstride = kv.k_bstride; e.k_hstride = kv.k_hstride; e.v = nullptr;
-  e.vt = w.vt; e.vt_ld = Sp; e.tap = qkv_tap;
+  e.k = kv.k; e.k_bstride = kv.k_bstride; e.k_hstride = kv.k_hstride;
+  e.v = kv.v; e.v_bstride = kv.v_bstride; e.v_hstride = kv.v_hstride; e.tap = qkv_tap;
   HIP_TRY(gemm_qkv(m->layers[layer].wqkv, (const f16*)xnorm, c.q_dim + 2 * c.kv_dim, T, c.dim, e, st));
-  TRY(zero_vt_pad(m, w.vt, B, S, st));
   AttnPrefill a{};
   a.q = w.q; a.q_rows = Sp; a.k = kv.k; a.k_bstride = kv.k_bstride; a.k_hstride = kv.k_hstride;
-  a.vt = w.vt; a.vt_ld = Sp; a.out = (f16*)attn; a.B = B; a.S = S; a.H = c.heads;
+  a.v = kv.v; a.v_bstride = kv.v_bstride; a.v_hstride = kv.v_hstride; a.out = (f16*)attn; a.B = B; a.S = S; a.H = c.heads;
   a.KVH = c.kv_heads; a.hd = c.hd; a.scale = 1.0f / sqrtf((float)c.hd);
   HIP_TRY(attention_prefill(a, st));
   return HB_OK;
@@ -2367,7 +2345,7 @@ int enqueue_decode_layer_split(hb_kv* kv, int l, const KVTarget& t, hipStream_t 
   e.kv_heads = c.kv_heads; e.rope = m->rope; e.rope_ld = m->rope_len; e.d_pos = kv->d_pos;
   e.q = kv->qd; e.q_rows = 1;
   e.k = t.k; e.k_bstride = t.k_bstride; e.k_hstride = t.k_hstride;
-  e.v = t.v; e.v_bstride = t.v_bstride; e.v_hstride = t.v_hstride; e.vt = nullptr; e.vt_ld = 0;
+  e.v = t.v; e.v_bstride = t.v_bstride; e.v_hstride = t.v_hstride;
   e.tap = nullptr;
   e.q_lo = kv->qd_lo; e.k_lo = t.k_lo; e.v_lo = t.v_lo;
   HIP_TRY(gemv_qkv(L.t_wqkv, kv->xn, nullptr, c.q_dim + 2 * c.kv_dim, B, c.dim, e, st, true));
@@ -2423,7 +2401,7 @@ int enqueue_decode_step(hb_kv* kv, hipStream_t st) {
     e.kv_heads = c.kv_heads; e.rope = m->rope; e.rope_ld = m->rope_len; e.d_pos = kv->d_pos;
     e.q = kv->qd; e.q_rows = 1;
     e.k = t.k; e.k_bstride = t.k_bstride; e.k_hstride = t.k_hstride;
-    e.v = t.v; e.v_bstride = t.v_bstride; e.v_hstride = t.v_hstride; e.vt = nullptr; e.vt_ld = 0;
+    e.v = t.v; e.v_bstride = t.v_bstride; e.v_hstride = t.v_hstride;
     e.tap = nullptr;
     HIP_TRY(gemv_qkv(L.t_wqkv, kv->xn, fused ? &n1 : nullptr, c.q_dim + 2 * c.kv_dim, B, c.dim, e, st,
                      false, xfrag));
@@ -2806,7 +2784,7 @@ int train_buffers(hb_model* m, int B, int S) {
   const size_t o_d16 = take(T * d * 2), o_d16T = take(d * Tp * 2), o_dh = take(T * 2 * h * 2),
                o_dhT = take(2 * h * Tp * 2), o_actT = take(actw * Tp * 2), o_dqkv = take(T * qkv * 2),
                o_dqkvT = take(qkv * Tp * 2), o_dl = take(T * Vp * 2), o_dlT = take(V * Tp * 2);
-  const size_t o_dA = take(qh * 2), o_vt = take(kvh * 2);
+  const size_t o_dA = take(qh * 2);
   hipStream_t st = m->ctx->stream();
   if (off > ts->abytes) {
     HIP_TRY(hipStreamSynchronize(st));
@@ -2835,7 +2813,7 @@ int train_buffers(hb_model* m, int B, int S) {
   ts->d16 = (f16*)(b + o_d16); ts->d16T = (f16*)(b + o_d16T); ts->dh = (f16*)(b + o_dh);
   ts->dhT = (f16*)(b + o_dhT); ts->actT = (f16*)(b + o_actT); ts->dqkv = (f16*)(b + o_dqkv);
   ts->dqkvT = (f16*)(b + o_dqkvT); ts->dl = (f16*)(b + o_dl); ts->dlT = (f16*)(b + o_dlT);
-  ts->dA = (f16*)(b + o_dA); ts->vt = (f16*)(b + o_vt);
+  ts->dA = (f16*)(b + o_dA);
   HIP_TRY(fill_f16_zero((f16*)b, off / 2, st));
   ts->B = B;
   ts->S = S;
@@ -2864,11 +2842,11 @@ int train_forward(hb_model* m, int B, int S) {
     e.q = A.q; e.q_rows = Sp;
     e.k = A.k; e.k_bstride = kbs; e.k_hstride = khs;
     e.v = A.v; e.v_bstride = kbs; e.v_hstride = khs;
-    e.vt = ts->vt; e.vt_ld = Sp; e.tap = nullptr;
+    e.tap = nullptr;
     HIP_TRY(gemm_qkv(L.wqkv, A.xn, qkv, T, c.dim, e, st));
     AttnPrefill a{};
     a.q = A.q; a.q_rows = Sp; a.k = A.k; a.k_bstride = kbs; a.k_hstride = khs;
-    a.vt = ts->vt; a.vt_ld = Sp; a.out = A.attn; a.B = B; a.S = S; a.H = c.heads;
+    a.v = A.v; a.v_bstride = kbs; a.v_hstride = khs; a.out = A.attn; a.B = B; a.S = S; a.H = c.heads;
     a.KVH = c.kv_heads; a.hd = c.hd; a.scale = 1.0f / sqrtf((float)c.hd); a.lse = A.lse;
     HIP_TRY(attention_prefill(a, st));
     GemmScratch so, s2;

@@ -95,6 +95,16 @@ HB_DEV void raw_barrier() {
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("" ::: "memory");
 }
+// Waits for the loads that fill v here. Registers loaded before a loop of
+// copies must be settled before it: the compiler otherwise waits for them at
+// their first use inside the loop, in every iteration, and that wait drains
+// the copies in flight with them.
+template <class V, int N>
+HB_DEV void settle(V (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
+}
+
 // LDS byte address of a __shared__ object, for dma_1k.
 template <class T>
 HB_DEV uint32_t lds_addr(T* p) {

@@ -164,16 +164,13 @@ struct EpiQKV {
   // K rows [s][hd] at k + b*k_bstride + kvh*k_hstride
   f16* k;
   size_t k_bstride, k_hstride;
-  // V rows [s][hd] (KV cache layout), nullable
+  // V rows [s][hd], as K
   f16* v;
   size_t v_bstride, v_hstride;
-  // V transposed [hd][s] for prefill attention: vt + (b*kv_heads+kvh)*hd*vt_ld, nullable
-  f16* vt;
-  int vt_ld;
   float* tap;  // nullable [T, q+2kv] fp32 = Q_rope | K_rope | V
   // Low parts of the two-term fp16 form (common.hpp) in the same layouts as
-  // q, k, v and vt; all NULL for plain fp16 outputs.
-  f16 *q_lo = nullptr, *k_lo = nullptr, *v_lo = nullptr, *vt_lo = nullptr;
+  // q, k and v; all NULL for plain fp16 outputs.
+  f16 *q_lo = nullptr, *k_lo = nullptr, *v_lo = nullptr;
   FastDiv div_S, div_hd;  // by S and hd; set by prepare() on the host
 
   __host__ void prepare() {
@@ -217,11 +214,11 @@ struct EpiQKV {
     return a;
   }
   // Output modes of the kernels' instances (EpiQKVAt): PLAIN writes fp16 Q,
-  // K and V^T and/or V rows (every layer but the two-term ones); SPLIT also
-  // writes the low parts (q_lo .. vt_lo); FULL also the fp32 tap.
+  // K and V rows (every layer but the two-term ones); SPLIT also
+  // writes the low parts (q_lo .. v_lo); FULL also the fp32 tap.
   enum Mode { PLAIN = 0, SPLIT = 1, FULL = 2 };
   __host__ int mode() const {
-    return tap ? FULL : (q_lo || k_lo || v_lo || vt_lo) ? SPLIT : PLAIN;
+    return tap ? FULL : (q_lo || k_lo || v_lo) ? SPLIT : PLAIN;
   }
   template <bool DEC, int MODE>
   HB_DEV void store_at(int t, int f0, f32x4 v4, const Aux& a, int fb) const {
@@ -242,22 +239,14 @@ struct EpiQKV {
     }
     const f16x4 oh = f16x4_hi(o);
     if constexpr (MODE == PLAIN) {
-      // one f16x4 store per quad (Q, K or V rows) and, for V^T, four
-      // 2-byte stores; every branch is wave-uniform (fb)
+      // one f16x4 store per quad; every branch is wave-uniform (fb)
       if (r0 == 0) {
         const size_t hs = (size_t)q_rows * hd;
         *(f16x4*)(q + b * (heads * hs) + h * hs + (size_t)(DEC ? 0 : s) * hd + e) = oh;
       } else if (r0 == q_dim) {
         *(f16x4*)(k + b * k_bstride + h * k_hstride + (size_t)s * hd + e) = oh;
       } else {
-        if (v) *(f16x4*)(v + b * v_bstride + h * v_hstride + (size_t)s * hd + e) = oh;
-        if (vt) {
-          f16* p = vt + ((size_t)b * kv_heads + h) * hd * vt_ld + (size_t)e * vt_ld + s;
-          p[0] = oh.x;
-          p[vt_ld] = oh.y;
-          p[2 * vt_ld] = oh.z;
-          p[3 * vt_ld] = oh.w;
-        }
+        *(f16x4*)(v + b * v_bstride + h * v_hstride + (size_t)s * hd + e) = oh;
       }
       return;
     }
@@ -283,25 +272,8 @@ struct EpiQKV {
       hs = v_hstride;
     }
     const size_t off = b * bs + h * hs + (size_t)srow * hd + e;
-    if (base) *(f16x4*)(base + off) = oh;
-    const bool lo = base_lo || (r0 == q_dim + kv_dim && vt_lo);
-    const f16x4 ol = lo ? f16x4_lo(o, oh) : f16x4{};
-    if (base_lo) *(f16x4*)(base_lo + off) = ol;
-    if (r0 == q_dim + kv_dim && vt) {
-      const size_t vo = ((size_t)b * kv_heads + h) * hd * vt_ld + (size_t)e * vt_ld + s;
-      f16* p = vt + vo;
-      p[0] = oh.x;
-      p[vt_ld] = oh.y;
-      p[2 * vt_ld] = oh.z;
-      p[3 * vt_ld] = oh.w;
-      if (vt_lo) {
-        f16* pl = vt_lo + vo;
-        pl[0] = ol.x;
-        pl[vt_ld] = ol.y;
-        pl[2 * vt_ld] = ol.z;
-        pl[3 * vt_ld] = ol.w;
-      }
-    }
+    *(f16x4*)(base + off) = oh;
+    if (base_lo) *(f16x4*)(base_lo + off) = f16x4_lo(o, oh);
     if (tap) *(f32x4*)(tap + (size_t)t * (q_dim + 2 * kv_dim) + f0) = o;
   }
 };
@@ -366,9 +338,8 @@ struct EpiQKVAt : EpiQKV {
     int b, s;
   };
   struct Row {
-    f16* p;   // row (b, s) of head h in the block's region (Q, K or V), at feature 0
-    f16* pt;  // column s of head h in V^T (V region)
-    int e0;   // feature of fb within its head
+    f16* p;  // row (b, s) of head h in the block's region (Q, K or V), at feature 0
+    int e0;  // feature of fb within its head
   };
   HB_DEV Tok tok(int t) const {
     Tok r;
@@ -377,14 +348,13 @@ struct EpiQKVAt : EpiQKV {
   }
   HB_DEV Row row(const Tok& tk, int fb) const {
     const int r0 = region_start(fb), fr = fb - r0, h = div_hd.div(fr);
-    Row r{nullptr, nullptr, fr - h * hd};
+    Row r{nullptr, fr - h * hd};
     if (r0 == 0) {
       r.p = q + ((size_t)tk.b * heads + h) * q_rows * hd + (size_t)tk.s * hd;
     } else if (r0 == q_dim) {
       r.p = k + tk.b * k_bstride + h * k_hstride + (size_t)tk.s * hd;
     } else {
-      if (v) r.p = v + tk.b * v_bstride + h * v_hstride + (size_t)tk.s * hd;
-      if (vt) r.pt = vt + ((size_t)tk.b * kv_heads + h) * hd * vt_ld + tk.s;
+      r.p = v + tk.b * v_bstride + h * v_hstride + (size_t)tk.s * hd;
     }
     return r;
   }
@@ -397,15 +367,7 @@ struct EpiQKVAt : EpiQKV {
       o.z = v4.z * a.c1.x - v4.w * a.c1.y;
       o.w = v4.w * a.c1.x + v4.z * a.c1.y;
     }
-    const f16x4 oh = f16x4_hi(o);
-    if (r0 < q_dim + kv_dim || v) *(f16x4*)(r.p + e) = oh;
-    if (r0 == q_dim + kv_dim && vt) {
-      f16* p = r.pt + (size_t)e * vt_ld;
-      p[0] = oh.x;
-      p[vt_ld] = oh.y;
-      p[2 * vt_ld] = oh.z;
-      p[3 * vt_ld] = oh.w;
-    }
+    *(f16x4*)(r.p + e) = f16x4_hi(o);
   }
   HB_DEV Aux load(int t, int f0) const { return load(t, f0, f0 & ~31); }
   HB_DEV void operator()(int t, int f0, f32x4 v4) const { (*this)(t, f0, v4, load(t, f0), f0 & ~31); }

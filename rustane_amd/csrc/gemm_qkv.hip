@@ -1,4 +1,4 @@
-// Prefill QKV projection (RoPE, head-major Q/K, V and V^T epilogue).
+// Prefill QKV projection (RoPE, head-major Q, K and V epilogue).
 #include "gemm_launch.hpp"
 
 namespace hb {

@@ -119,14 +119,14 @@ struct AttnPrefill {
   int q_rows;
   const f16* k;  // rows [s][hd] at k + b*k_bstride + kvh*k_hstride
   size_t k_bstride, k_hstride;
-  const f16* vt;  // [B][KVH][hd][vt_ld]
-  int vt_ld;
+  const f16* v;  // rows [s][hd] at v + b*v_bstride + kvh*v_hstride
+  size_t v_bstride, v_hstride;
   f16* out;  // [B*S][H*hd], or split rows [B*S][2*H*hd] when q_lo is set
   int B, S, H, KVH, hd;
   float scale;  // 1/sqrt(hd)
-  // Two-term fp16 inputs (common.hpp): low parts of q, k and vt in the same
+  // Two-term fp16 inputs (common.hpp): low parts of q, k and v in the same
   // layouts, all set or all NULL.
-  const f16 *q_lo = nullptr, *k_lo = nullptr, *vt_lo = nullptr;
+  const f16 *q_lo = nullptr, *k_lo = nullptr, *v_lo = nullptr;
   // Training: per-query log-sum-exp of the scaled scores in log2 units,
   // lse[(b*H + h)*q_rows + s] = log2(sum_t exp2(sc[s,t] * scale * log2 e)),
   // for the fused backward. NULL: not written.

@@ -288,6 +288,36 @@ def test_sdpa_plain_stores_equal_tapped(gpu, B, S):
     k.ctx.close()
 
 
+@pytest.mark.parametrize("hd,heads,kv", [(128, 4, 2), (64, 4, 4)])
+@pytest.mark.parametrize("S", [1, 31, 33, 250])
+def test_sdpa_ignores_stale_rows_past_the_sequence(gpu, S, hd, heads, kv):
+    """The K and V rows between S and the next multiple of 32 keep what an
+    earlier, longer call left there: infinities and NaN from it must not reach
+    a shorter sequence, whose output equals a fresh model's bit for bit."""
+    import torch
+    cfg = tiny_config(dim=512, hidden=256, heads=heads, kv_heads=kv, hd=hd, nlayers=1, seq=256, vocab=256)
+    w = ModelWeights.synthetic(cfg, seed=79, std=0.02)
+    xn = to_dev(f16_round(np.random.default_rng(13).standard_normal((S, cfg.dim))), torch.float16)
+    bad = torch.full((cfg.seq, cfg.dim), float("inf"), dtype=torch.float16, device="cuda")
+    print(f"sdpa stale rows: S={S} hd={hd} heads={heads}/{kv}", flush=True)
+    outs = []
+    for spoil in (False, True):
+        k = CompiledKernels.compile(cfg)
+        k.ctx.set_stream(gpu.stream())
+        k.ensure_weights(w)
+        if spoil:
+            scrap = torch.empty((cfg.seq, cfg.q_dim), dtype=torch.float16, device="cuda")
+            hb.call("hb_op_sdpa_fwd", k.model.handle, 0, bad.data_ptr(), 1, cfg.seq, scrap.data_ptr(), None)
+        out = torch.empty((S, cfg.q_dim), dtype=torch.float16, device="cuda")
+        hb.call("hb_op_sdpa_fwd", k.model.handle, 0, xn.data_ptr(), 1, S, out.data_ptr(), None)
+        torch.cuda.synchronize()
+        outs.append(out.cpu().numpy())
+        k.model.close()
+        k.ctx.close()
+    assert np.isfinite(outs[0].astype(F32)).all()
+    np.testing.assert_array_equal(outs[0].view(np.uint16), outs[1].view(np.uint16))
+
+
 def test_logits_ce_op_matches_oracle(tiny):
     import torch
     cfg, k, w = tiny
