@@ -335,12 +335,27 @@ hipError_t attention_prefill(const AttnPrefill& p, hipStream_t st) {
 // GEMV prologue (gemv.hip) when B * chunks is small -- or by
 // attn_combine_kernel below, which folds them in the same order with the
 // same arithmetic, so both give the same attention output.
+//
+// Few heads (B x H <= 16): the launch is VALU work of few workgroups (16
+// waves, each block of 512 keys run by quarters), so chunks of 256 keys are
+// taken while the Wo prologue can still merge them all; from 4096 keys of
+// capacity the general rule gives as many. 12 heads at 1000 keys in 5 chunks
+// instead of 3: 7.1 -> 5.8 us, Wo 4.3 -> 4.5 us.
+//
+// What bounds it at a few hundred keys per workgroup: fp32 VALU issue, four
+// waves to a SIMD. Running only the quarters that hold keys, v_dot2 for the
+// scores and a merge by HD threads instead of all took 12 heads of 128 at
+// 1000 keys from 8.2 to 7.1 us (5.8 with the chunks above), and a step of
+// eight 64-wide heads at 64 keys x 8 layers from 212 to 172 us with the norm
+// prologue's (gemv.hip).
 constexpr int DMIN_CHUNK = 512;  // fewest keys of ctx_max per chunk
+constexpr int DFEW_HEADS = 16, DFEW_CHUNK = 256;
 
 AttnChunking attn_decode_chunking(int ctx_max, int B, int H) {
   const int bh = std::max(1, B * H);
   const int most = std::max(1, (ctx_max + DMIN_CHUNK - 1) / DMIN_CHUNK);
-  const int n = std::max(1, std::min(most, 256 / bh));
+  int n = std::max(1, std::min(most, 256 / bh));
+  if (bh <= DFEW_HEADS) n = std::max(n, std::min((ctx_max + DFEW_CHUNK - 1) / DFEW_CHUNK, GEMV_ATTN_MAXCH / B));
   return AttnChunking{n, n == 1 && bh >= 256 ? 8 : 16};
 }
 
@@ -348,7 +363,7 @@ AttnChunking attn_decode_chunking(int ctx_max, int B, int H) {
 // fp32 as they are loaded (the arithmetic is fp32 throughout).
 template <int HD, bool SPLIT, int NW>
 __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(AttnDecode p) {
-  constexpr int NT = NW * 64;
+  static_assert(NW * 64 >= HD, "one thread per element of the merge");
   constexpr int LPK = HD / 8;       // lanes per key row
   constexpr int KPW = 64 / LPK;     // keys per wave instruction
   constexpr int STRIPE = NW * KPW;  // keys per instruction of all waves
@@ -369,10 +384,10 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(AttnDecode p) {
 
   const size_t qo = ((size_t)b * p.H + h) * HD + 8 * j;
   const f16x8 qv = *(const f16x8*)(p.q + qo);
-  float qf[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) qf[i] = (float)qv[i];
+  float qf[8];  // SPLIT only
   if constexpr (SPLIT) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) qf[i] = (float)qv[i];
     const f16x8 ql = *(const f16x8*)(p.q_lo + qo);
 #pragma unroll
     for (int i = 0; i < 8; ++i) qf[i] += (float)ql[i];
@@ -384,13 +399,14 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(AttnDecode p) {
 
   // Online softmax state of this lane's keys (m is wave-uniform).
   float m = -INFINITY, l = 0.f, acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int b0 = c0; b0 < cend; b0 += BLOCK) {
+  auto block = [&](auto nc, int b0) {  // the block's first NI instructions
+    constexpr int NI = decltype(nc)::value;
     const int kbase = b0 + wave * KPW + g;  // key of instruction i: kbase + i * STRIPE
-    constexpr int NL = SPLIT ? NIT : 1;
-    f16x8 kr[NIT], krl[NL];
+    constexpr int NL = SPLIT ? NI : 1;
+    f16x8 kr[NI], krl[NL];
     const f16x8 zero8 = {};
 #pragma unroll
-    for (int i = 0; i < NIT; ++i) {
+    for (int i = 0; i < NI; ++i) {
       const int kk = kbase + i * STRIPE;
       kr[i] = kk < cend ? __builtin_nontemporal_load((const f16x8*)(kb + (size_t)kk * HD)) : zero8;
       if constexpr (SPLIT)
@@ -399,7 +415,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(AttnDecode p) {
     // Without low parts the V loads go out with K's, before the scores. With
     // them they follow the scores, in two halves, so that K's registers are
     // free again and one half of V (hi and lo) is live at a time.
-    constexpr int NV = SPLIT ? NIT / 2 : NIT;
+    constexpr int NV = SPLIT ? NI / 2 : NI;
     f16x8 vr[NV], vrl[SPLIT ? NV : 1];
     auto load_v = [&](int i0) {
 #pragma unroll
@@ -411,20 +427,25 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(AttnDecode p) {
       }
     };
     if constexpr (!SPLIT) load_v(0);
-    auto kval = [&](int i, int e) { return SPLIT ? (float)kr[i][e] + (float)krl[i % NL][e] : (float)kr[i][e]; };
-    float sc[NIT];
+    float sc[NI];
 #pragma unroll
-    for (int i = 0; i < NIT; ++i) {
+    for (int i = 0; i < NI; ++i) {
       float d = 0.f;
+      if constexpr (SPLIT) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) d += qf[e] * kval(i, e);
+        for (int e = 0; e < 8; ++e) d += qf[e] * ((float)kr[i][e] + (float)krl[i][e]);
+      } else {  // exact fp16 products summed in fp32
+#pragma unroll
+        for (int e = 0; e < 8; e += 2)
+          d = __builtin_amdgcn_fdot2(f16x2{qv[e], qv[e + 1]}, f16x2{kr[i][e], kr[i][e + 1]}, d, false);
+      }
       d = group_sum<LPK>(d);
       sc[i] = (kbase + i * STRIPE < cend) ? d * sl2 : -INFINITY;
     }
     // wave-wide max over this block's keys (lanes of a group hold equal scores)
     float mb = sc[0];
 #pragma unroll
-    for (int i = 1; i < NIT; ++i) mb = fmaxf(mb, sc[i]);
+    for (int i = 1; i < NI; ++i) mb = fmaxf(mb, sc[i]);
     mb = fold_groups<LPK>(mb, [](float a, float c) { return fmaxf(a, c); });
     const float mn = fmaxf(m, mb);
     if (mn != -INFINITY) {
@@ -436,7 +457,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(AttnDecode p) {
         m = mn;
       }
 #pragma unroll
-      for (int i0 = 0; i0 < NIT; i0 += NV) {
+      for (int i0 = 0; i0 < NI; i0 += NV) {
         if constexpr (SPLIT) load_v(i0);
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
@@ -452,6 +473,20 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(AttnDecode p) {
         }
       }
     }
+  };
+  for (int b0 = c0; b0 < cend; b0 += BLOCK) {
+    // Quarters of the block that hold keys; each count has its own
+    // straight-line code, so that all its loads still go out together. With
+    // low parts the block is run whole (its registers are at the limit).
+    const int nq = SPLIT ? 4 : (cend - b0 + BLOCK / 4 - 1) / (BLOCK / 4);
+    if (!SPLIT && nq <= 1)
+      block(std::integral_constant<int, SPLIT ? NIT : NIT / 4>{}, b0);
+    else if (!SPLIT && nq == 2)
+      block(std::integral_constant<int, SPLIT ? NIT : NIT / 2>{}, b0);
+    else if (!SPLIT && nq == 3)
+      block(std::integral_constant<int, SPLIT ? NIT : NIT * 3 / 4>{}, b0);
+    else
+      block(std::integral_constant<int, NIT>{}, b0);
   }
   {
     const auto add = [](float a, float c) { return a + c; };
@@ -468,46 +503,42 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(AttnDecode p) {
     for (int e = 0; e < 8; ++e) s_o[wave][8 * j + e] = acc[e];
   }
   __syncthreads();
+  // The merge of NW partials is ~10 instructions per partial and only HD
+  // threads have an element: the other waves leave the SIMDs to them.
+  if (tid >= HD) return;
   float M = s_m[0];
 #pragma unroll
   for (int v = 1; v < NW; ++v) M = fmaxf(M, s_m[v]);
   // Wave weights exp2(m_w - M); a wave whose keys are all past the chunk has
   // m_w = -inf and weight 0.
-  auto wt = [&](int v) { return s_m[v] == -INFINITY ? 0.f : exp2f(s_m[v] - M); };
-  float L = 0.f;
+  float wt[NW], L = 0.f, o = 0.f;
 #pragma unroll
-  for (int v = 0; v < NW; ++v) L += wt(v) * s_l[v];
+  for (int v = 0; v < NW; ++v) {
+    wt[v] = s_m[v] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[v] - M);
+    L += wt[v] * s_l[v];
+    o += wt[v] * s_o[v][tid];
+  }
+  const int e = tid;
   const size_t head = (size_t)b * p.H + h;
   if (gridDim.x == 1) {
     // One chunk: the normalised attention row, fp16 (split rows [B][2*H*hd]
     // hi | lo with two-term inputs), as attention_combine would write it.
-    const float iL = 1.0f / L;
-    for (int e = tid; e < HD; e += NT) {
-      float o = 0.f;
-#pragma unroll
-      for (int v = 0; v < NW; ++v) o += wt(v) * s_o[v][e];
-      o *= iL;
-      const f16 hi = (f16)o;
-      if (p.q_lo) {
-        f16* op = p.out + (size_t)b * 2 * p.H * HD + h * HD + e;
-        op[0] = hi;
-        op[(size_t)p.H * HD] = (f16)(o - (float)hi);
-      } else if (p.out_frag) {  // the Wo GEMV's B-fragment order over K = H*hd
-        const int k = h * HD + e;
-        p.out[((size_t)(k >> 5) * 64 + b + 16 * ((k & 31) >> 3)) * 8 + (k & 7)] = hi;
-      } else {
-        p.out[head * HD + e] = hi;
-      }
+    o *= 1.0f / L;
+    const f16 hi = (f16)o;
+    if (p.q_lo) {
+      f16* op = p.out + (size_t)b * 2 * p.H * HD + h * HD + e;
+      op[0] = hi;
+      op[(size_t)p.H * HD] = (f16)(o - (float)hi);
+    } else if (p.out_frag) {  // the Wo GEMV's B-fragment order over K = H*hd
+      const int k = h * HD + e;
+      p.out[((size_t)(k >> 5) * 64 + b + 16 * ((k & 31) >> 3)) * 8 + (k & 7)] = hi;
+    } else {
+      p.out[head * HD + e] = hi;
     }
     return;
   }
   const size_t slot = head * gridDim.x + blockIdx.x;
-  for (int e = tid; e < HD; e += NT) {
-    float o = 0.f;
-#pragma unroll
-    for (int v = 0; v < NW; ++v) o += wt(v) * s_o[v][e];
-    p.part_o[slot * HD + e] = o;
-  }
+  p.part_o[slot * HD + e] = o;
   if (tid == 0) {
     p.part_ml[slot * 2] = M;
     p.part_ml[slot * 2 + 1] = L;

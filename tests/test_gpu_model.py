@@ -280,6 +280,25 @@ def test_decode_long_context_both_chunk_combines(m48):
         assert int(n3[0]) == int(n1[0])
 
 
+@pytest.mark.parametrize("B, ctx", [(1, 256), (1, 2048), (2, 1024), (4, 512), (8, 1024)])
+def test_decode_rows_at_attention_block_edges(m48, B, ctx):
+    """Decode attention runs the quarters (128 keys of a 64-wide head) of a
+    512-key block that hold keys: one step at positions on both sides of each
+    quarter's and block's edge, in 1 to 8 chunks, at the row counts of the norm
+    prologue (1, 2, up to 8), against the prefill of one token more. Both
+    sides are within ~1e-3 of the oracle on this model."""
+    cfg, w, k = m48
+    a, b = E.Decoder(k, batch=B, ctx_max=ctx), E.Decoder(k, batch=B, ctx_max=ctx)
+    for P in [p for p in (1, 63, 127, 128, 255, 256, 383, 384, 511, 512, 1000) if p < ctx]:
+        tok = tokens_for(cfg, B * (P + 1), seed=91 + P).reshape(B, P + 1)
+        a.kv.reset()
+        b.kv.reset()
+        a.prefill(tok[:, :P])
+        got, _ = a.step(tok[:, P])
+        ref, _ = b.prefill(tok)
+        assert np.abs(got - ref).max() < 2e-3, P
+
+
 def test_error_paths(gpu):
     cfg = tiny_config()
     k = CompiledKernels.compile(cfg)
