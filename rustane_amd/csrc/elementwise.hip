@@ -236,6 +236,41 @@ hipError_t set_int(int* d, int value, hipStream_t st) {
   return hipGetLastError();
 }
 
+// ---- decode step input and output -------------------------------------------------
+// The step's tokens travel in the kernel's arguments, its results by stores
+// to the cache's pinned host buffer: a copy command between kernels costs
+// 10-20 us of queue and host time, as much as several of the step's launches.
+// 128 workgroups keep PCIe full (2 MB of logits ~40 us).
+__global__ void decode_begin_kernel(DecodeTokens t, int B, uint32_t* d_tok, int* d_pos0, int pos0) {
+  if ((int)threadIdx.x < B) d_tok[threadIdx.x] = t.id[threadIdx.x];
+  if (threadIdx.x == 0) *d_pos0 = pos0;
+}
+hipError_t decode_begin(const DecodeTokens& t, int B, uint32_t* d_tok, int* d_pos0, int pos0, hipStream_t st) {
+  if (B < 1 || B > 16) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(decode_begin_kernel, dim3(1), dim3(64), 0, st, t, B, d_tok, d_pos0, pos0);
+  return hipGetLastError();
+}
+
+__global__ __launch_bounds__(256) void decode_publish_kernel(const float* __restrict__ logits, size_t n4,
+                                                             const uint32_t* __restrict__ next, int B,
+                                                             const int* __restrict__ err, DecodeHost* __restrict__ h) {
+  f32x4* const out = (f32x4*)h->logits();
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256)
+    out[i] = ((const f32x4*)logits)[i];
+  if (blockIdx.x == 0) {
+    if ((int)threadIdx.x < B) h->next[threadIdx.x] = next[threadIdx.x];
+    if (threadIdx.x == 0) h->err = *err;
+  }
+}
+hipError_t decode_publish(const float* logits, size_t n, const uint32_t* next, int B, const int* err, DecodeHost* h,
+                          hipStream_t st) {
+  if (n % 4 || B < 1 || B > 16) return hipErrorInvalidValue;
+  const size_t n4 = n / 4;
+  const int grid = (int)std::max<size_t>(1, std::min<size_t>((n4 + 255) / 256, 128));
+  hipLaunchKernelGGL(decode_publish_kernel, dim3(grid), dim3(256), 0, st, logits, n4, next, B, err, h);
+  return hipGetLastError();
+}
+
 // ---- weight repacking -------------------------------------------------------------
 HB_DEV int repack_row(int mode, int i, int j, int row0) {
   if (mode == 0) return row0 + j;

@@ -206,6 +206,20 @@ hipError_t cross_entropy(const float* logits, const uint32_t* targets, int T, in
                          float* loss, int* err, hipStream_t st);
 hipError_t mean_reduce(const float* v, int n, float* out, hipStream_t st);
 hipError_t set_int(int* d, int value, hipStream_t st);
+// A decode step's tokens, by value; what a step or prefill returns, in pinned
+// host memory, the logits behind it. decode_publish writes n logits (n = 0:
+// none), the next tokens and the error word there.
+struct DecodeTokens {
+  uint32_t id[16];
+};
+struct alignas(128) DecodeHost {
+  int err;
+  uint32_t next[16];
+  __host__ __device__ float* logits() { return (float*)(this + 1); }
+};
+hipError_t decode_begin(const DecodeTokens& t, int B, uint32_t* d_tok, int* d_pos0, int pos0, hipStream_t st);
+hipError_t decode_publish(const float* logits, size_t n, const uint32_t* next, int B, const int* err, DecodeHost* h,
+                          hipStream_t st);
 
 // Weight repacking: src fp32 [R][C] row-major (device), dst fp16.
 //   mode 0: dst[(row0 + j) * ld + i] = src[i][j]              (transpose)

@@ -299,6 +299,34 @@ def test_decode_rows_at_attention_block_edges(m48, B, ctx):
         assert np.abs(got - ref).max() < 2e-3, P
 
 
+@pytest.mark.parametrize("B", [1, 5, 16])
+def test_decode_results_reach_any_buffer(m48, B):
+    """A step's and a prefill's results come through the cache's pinned buffer:
+    into an unaligned part of a larger array without touching its neighbours,
+    and with either result left out, the same values as through Decoder."""
+    cfg, w, k = m48
+    n, P = B * cfg.vocab, 3
+    tok = tokens_for(cfg, B * (P + 1), seed=17).reshape(B, P + 1)
+    prompt, last = np.ascontiguousarray(tok[:, :P]).reshape(-1), np.ascontiguousarray(tok[:, P])
+    ref = E.Decoder(k, batch=B, ctx_max=P + 1)
+    want = ref.prefill(prompt), ref.step(last)
+    dec = E.Decoder(k, batch=B, ctx_max=P + 1)
+    for logits, nxt in ((True, True), (False, True), (True, False), (False, False)):
+        buf, ids = np.full(n + 7, 3.25, np.float32), np.full(B + 2, 77, np.uint32)
+        args = (hb.ptr(buf[3:3 + n]) if logits else None, hb.ptr(ids[1:1 + B]) if nxt else None)
+        dec.kv.reset()
+        for call, ref_out in ((("hb_prefill", prompt, P), want[0]), (("hb_decode_step", last), want[1])):
+            buf[:], ids[:] = 3.25, 77
+            hb.call(call[0], k.model.handle, dec.kv.handle, hb.ptr(call[1]), *call[2:], *args)
+            exp, exp_ids = np.full(n + 7, 3.25, np.float32), np.full(B + 2, 77, np.uint32)
+            if logits:
+                exp[3:3 + n] = ref_out[0].reshape(-1)
+            if nxt:
+                exp_ids[1:1 + B] = ref_out[1]
+            np.testing.assert_array_equal(buf, exp)
+            np.testing.assert_array_equal(ids, exp_ids)
+
+
 def test_error_paths(gpu):
     cfg = tiny_config()
     k = CompiledKernels.compile(cfg)
