@@ -327,6 +327,26 @@ def test_decode_results_reach_any_buffer(m48, B):
             np.testing.assert_array_equal(ids, exp_ids)
 
 
+@pytest.mark.parametrize("B, dim", [(3, 320), (4, 320), (9, 64), (16, 576)])
+def test_decode_precise_layer_wide_projections(gpu, B, dim):
+    """The two-term first layer with over 256 row blocks in QKV and W1|W3: from
+    4 sequences its GEMVs keep both halves of their rows in registers. dim / 32
+    k-steps over the 8 waves leave waves with none (64), 1 or 2 (320), 2 or 3
+    (576). One step against the prefill of one token more; both round to fp16
+    alike but for the order of fp32 sums."""
+    cfg = E.ModelConfig.make(dim=dim, hidden=2304, heads=22, nlayers=2, seq=40, vocab=256, hd=64)
+    k = CompiledKernels.compile(cfg)
+    k.init_synthetic(5, 0.02)
+    P = 33
+    tok = tokens_for(cfg, B * (P + 1), seed=19).reshape(B, P + 1)
+    a, b = E.Decoder(k, batch=B, ctx_max=P + 1), E.Decoder(k, batch=B, ctx_max=P + 1)
+    a.prefill(tok[:, :P])
+    got, _ = a.step(tok[:, P])
+    ref, _ = b.prefill(tok)
+    assert np.abs(ref).max() > 0.05
+    assert np.abs(got - ref).max() < 2e-3
+
+
 def test_error_paths(gpu):
     cfg = tiny_config()
     k = CompiledKernels.compile(cfg)
