@@ -207,7 +207,7 @@ int hb_model_reserve(hb_model* model, int B, int S);
  * the kernels between two HIP events on the stream:
  *   rmsnorm1_ms           the separate input norms (layer 0's; later layers'
  *                         come out of the previous W2 reduction, below)
- *   sdpa_qkv_ms           Q/K/V projection + RoPE + K/V^T scatter   (sdpaFwd)
+ *   sdpa_qkv_ms           Q/K/V projection + RoPE + K/V scatter     (sdpaFwd)
  *   sdpa_attention_ms     causal attention                          (sdpaFwd)
  *   wo_ms                 Wo projection (split-K partial sums)      (woFwd)
  *   residual_rmsnorm2_ms  split-K reduction + residual + RMSNorm2

@@ -13,7 +13,7 @@
 // registers 8j..8j+7 of lane half h2 hold the consecutive rows 16j+8h2..+7
 // and serve directly as a B operand. The same tile also gives the transposed
 // A operand (one feature, 8 consecutive rows) through ds_read_b64_tr_b16
-// (tr_frag), so no transposed copies exist in memory or LDS.
+// (TrFrag), so no transposed copies exist in memory or LDS.
 //
 // Tiles go from global memory straight into LDS (dma_1k) one or two
 // iterations ahead, with one barrier per iteration; a workgroup is 4 waves of
