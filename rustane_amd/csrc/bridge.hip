@@ -2481,33 +2481,38 @@ int launch_decode_step(hb_kv* kv) {
   return HB_OK;
 }
 
+// Whether the host itself may write a result buffer: device and managed
+// addresses take a runtime copy instead.
+bool host_writes(const void* p) {
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, p) == hipSuccess)
+    return at.type != hipMemoryTypeDevice && at.type != hipMemoryTypeManaged;
+  (void)hipGetLastError();  // plain memory that the runtime does not know
+  return true;
+}
+
 // Hands the results of the step or prefill that the stream holds to the
-// caller's buffers (nullable), waits for it and reports the error word. While
-// the device works, the host touches each page of the logits buffer, so that
-// a buffer fresh from the allocator takes its page faults then and not in the
-// copy (16 x 32000 logits: 340 us of faults a step).
+// caller's buffers (nullable, each host, device or managed memory), waits for
+// it and reports the error word. While the device works, the host touches each
+// page of a host logits buffer, so that a buffer fresh from the allocator
+// takes its page faults then and not in the copy (16 x 32000 logits: 340 us of
+// faults a step).
 int finish_decode(hb_kv* kv, float* h_logits, uint32_t* h_next) {
   hb_ctx* ctx = kv->model->ctx;
   hipStream_t st = ctx->stream();
-  const size_t n = (size_t)kv->B * kv->model->cfg.vocab;
-  bool direct = false;  // not plain host memory: the runtime copies
-  if (h_logits) {
-    hipPointerAttribute_t at{};
-    if (hipPointerGetAttributes(&at, h_logits) == hipSuccess)
-      direct = at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged;
-    else
-      (void)hipGetLastError();
-  }
-  HIP_TRY(decode_publish(kv->logits, h_logits && !direct ? n : 0, kv->d_next, kv->B, ctx->d_err, kv->host, st));
-  if (direct) HIP_TRY(hipMemcpyAsync(h_logits, kv->logits, n * 4, hipMemcpyDefault, st));
-  if (h_logits && !direct) {
+  const size_t n = (size_t)kv->B * kv->model->cfg.vocab, nb = (size_t)kv->B * 4;
+  const bool host_logits = h_logits && host_writes(h_logits), host_next = h_next && host_writes(h_next);
+  HIP_TRY(decode_publish(kv->logits, host_logits ? n : 0, kv->d_next, kv->B, ctx->d_err, kv->host, st));
+  if (h_logits && !host_logits) HIP_TRY(hipMemcpyAsync(h_logits, kv->logits, n * 4, hipMemcpyDefault, st));
+  if (h_next && !host_next) HIP_TRY(hipMemcpyAsync(h_next, kv->d_next, nb, hipMemcpyDefault, st));
+  if (host_logits) {
     volatile char* const p = (volatile char*)h_logits;
     for (size_t i = 0; i < n * 4; i += 4096) p[i] = p[i];
     p[n * 4 - 1] = p[n * 4 - 1];
   }
   HIP_TRY(hipStreamSynchronize(st));
-  if (h_logits && !direct) memcpy(h_logits, kv->host->logits(), n * 4);
-  if (h_next) memcpy(h_next, kv->host->next, (size_t)kv->B * 4);
+  if (host_logits) memcpy(h_logits, kv->host->logits(), n * 4);
+  if (host_next) memcpy(h_next, kv->host->next, nb);
   return report_err_word(ctx, kv->host->err);
 }
 

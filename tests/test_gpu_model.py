@@ -327,6 +327,48 @@ def test_decode_results_reach_any_buffer(m48, B):
             np.testing.assert_array_equal(ids, exp_ids)
 
 
+@pytest.mark.parametrize("kind", ["device", "pinned"])
+def test_decode_results_reach_device_and_pinned_buffers(m48, kind):
+    """Each of the two results may go to device memory (the runtime copies it)
+    or to pinned host memory, alone or together, into a slice whose neighbours
+    stay untouched, with the values that plain host arrays get."""
+    import torch
+    cfg, w, k = m48
+    B, P = 3, 4
+    n = B * cfg.vocab
+    tok = tokens_for(cfg, B * (P + 1), seed=23).reshape(B, P + 1)
+    prompt, last = np.ascontiguousarray(tok[:, :P]).reshape(-1), np.ascontiguousarray(tok[:, P])
+    ref = E.Decoder(k, batch=B, ctx_max=P + 1)
+    want = ref.prefill(prompt), ref.step(last)
+    dec = E.Decoder(k, batch=B, ctx_max=P + 1)
+    place = dict(device="cuda") if kind == "device" else dict(pin_memory=True)
+    for logits, nxt in ((True, True), (False, True), (True, False)):
+        dec.kv.reset()
+        for call, ref_out in ((("hb_prefill", prompt, P), want[0]), (("hb_decode_step", last), want[1])):
+            buf = torch.full((n + 7,), 3.25, **place)
+            ids = torch.full((B + 2,), 77, dtype=torch.int32, **place)
+            host_buf, host_ids = np.full(n, 3.25, np.float32), np.full(B, 77, np.uint32)
+            torch.cuda.synchronize()
+            print(f"decode results: {kind} {call[0]} logits={logits} next={nxt}", flush=True)
+            # the other of the two stays in a plain array
+            hb.call(call[0], k.model.handle, dec.kv.handle, hb.ptr(call[1]), *call[2:],
+                    buf[3:3 + n].data_ptr() if logits else hb.ptr(host_buf),
+                    ids[1:1 + B].data_ptr() if nxt else hb.ptr(host_ids))
+            torch.cuda.synchronize()
+            got, got_ids = buf.cpu().numpy(), ids.cpu().numpy().view(np.uint32)
+            exp, exp_ids = np.full(n + 7, 3.25, np.float32), np.full(B + 2, 77, np.uint32)
+            if logits:
+                exp[3:3 + n] = ref_out[0].reshape(-1)
+            else:
+                np.testing.assert_array_equal(host_buf, ref_out[0].reshape(-1))
+            if nxt:
+                exp_ids[1:1 + B] = ref_out[1]
+            else:
+                np.testing.assert_array_equal(host_ids, ref_out[1])
+            np.testing.assert_array_equal(got, exp)
+            np.testing.assert_array_equal(got_ids, exp_ids)
+
+
 @pytest.mark.parametrize("B, dim", [(3, 320), (4, 320), (9, 64), (16, 576)])
 def test_decode_precise_layer_wide_projections(gpu, B, dim):
     """The two-term first layer with over 256 row blocks in QKV and W1|W3: from
