@@ -65,21 +65,18 @@ HB_DEV i32x4 dma_rsrc(const void* base) {
 }
 // One wave copies 64 x 16 bytes from global memory (per-lane byte offset voff,
 // wave-uniform soff, both from the buffer's base) straight into LDS at
-// lds + 16 * lane. No output register;
-// the copy is counted by vmcnt (dma_wait). The nop is the wait state between
-// the write of m0 and its use.
+// lds + 16 * lane. No output register; the copy is counted by vmcnt
+// (dma_wait). The LDS address is an operand in m0, so that the compiler writes
+// that register itself and knows of it; the nop is the wait state between the
+// write of m0 and its use.
 HB_DEV void dma_1k(uint32_t lds, uint32_t voff, i32x4 rsrc, uint32_t soff) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc),
-      "s"(soff)
-      : "memory");
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+               : "memory");
 }
 // The same with 64 x 4 bytes.
 HB_DEV void dma_256(uint32_t lds, uint32_t voff, i32x4 rsrc, uint32_t soff) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc),
-      "s"(soff)
-      : "memory");
+  asm volatile("s_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+               : "memory");
 }
 // At most N of this wave's copies in flight; all its LDS reads done.
 template <int N>

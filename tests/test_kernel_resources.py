@@ -17,6 +17,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(ROOT, "rustane_amd", "libhip_bridge.so")
 LLVM = "/opt/rocm/llvm/bin"
+CSRC = os.path.join(ROOT, "rustane_amd", "csrc")
 
 
 def _kernel_metadata():
@@ -75,3 +76,21 @@ def test_kernels_fit_the_cu():
         assert int(k["group_segment_fixed_size"]) <= 160 * 1024, k["name"]
         assert int(k["vgpr_count"]) <= 512, k["name"]
         assert k.get("uses_dynamic_stack", "false") == "false", k["name"]
+
+
+def test_inline_asm_leaves_m0_to_the_compiler():
+    """m0 cannot be listed as clobbered (the compiler reserves it and warns),
+    so an asm block that writes it is invisible to code around it that uses it:
+    the direct-to-LDS copies take it as an operand instead."""
+    copies = 0
+    for name in sorted(os.listdir(CSRC)):
+        if not name.endswith((".hip", ".hpp")):
+            continue
+        text = open(os.path.join(CSRC, name)).read()
+        for stmt in re.findall(r"\basm\b[^;]*;", text):
+            template = "".join(re.findall(r'"((?:[^"\\]|\\.)*)"', stmt.split("::")[0]))
+            assert not re.search(r"\bm0\b", template), (name, template)
+            if re.search(r"buffer_load\w* .* lds\b", template):
+                copies += 1
+                assert '"{m0}"(' in stmt, (name, template)
+    assert copies >= 2, "expected the direct-to-LDS copies in the sources"
