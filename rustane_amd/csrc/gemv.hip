@@ -434,13 +434,29 @@ constexpr int GEMV_XREG_WGS = 256;
 constexpr int GEMV_XREG_U = 8;
 constexpr int GEMV_U = 4;   // 1 KB weight loads in flight per wave
 
+// X in split rows [B][2K]: the two-term layers' projections and the logits
+// behind them; no other epilogue's kernels are built for them.
+template <class Epi>
+hipError_t launch_gemv_split(const f16* Wt, const f16* X, int N, int B, int K, const Epi& epi, hipStream_t st) {
+  if (B < 1 || B > 16 || N % 16 || K % 32) return hipErrorInvalidValue;
+  if (B >= GEMV_XREG_MINB && K <= 32 * GEMV_XS * GEMV_KS && N / 16 > GEMV_XREG_WGS) {
+    const int nrb = N / 16, per = (nrb + GEMV_XREG_WGS - 1) / GEMV_XREG_WGS;
+    hipLaunchKernelGGL((gemv_xreg_kernel<GEMV_KS, GEMV_XS, GEMV_XREG_U, Epi, false, true>),
+                       dim3((nrb + per - 1) / per), dim3(GEMV_KS * 64), 0, st, (const f16x8*)Wt, X, N, B, K, epi);
+  } else {
+    hipLaunchKernelGGL((gemv_kernel<GEMV_KS, GEMV_U, Epi, PRO_NONE, true>), dim3(N / 16),
+                       dim3(GEMV_KS * 64), 0, st, (const f16x8*)Wt, X, N, B, K, epi, NormIn{},
+                       AttnIn{});
+  }
+  return hipGetLastError();
+}
+
 template <class Epi>
 hipError_t launch_gemv(const f16* Wt, const f16* X, const NormIn* nin, const AttnIn* ain, int N,
-                       int B, int K, const Epi& epi, hipStream_t st, bool split = false,
-                       bool xfrag = false) {
+                       int B, int K, const Epi& epi, hipStream_t st, bool xfrag) {
   if (B < 1 || B > 16 || N % 16 || K % 32) return hipErrorInvalidValue;
   if (xfrag) {  // X in B-fragment order (no prologue)
-    if (split || nin || ain) return hipErrorInvalidValue;
+    if (nin || ain) return hipErrorInvalidValue;
     if (K <= 32 * GEMV_XS * GEMV_KS && N / 16 > GEMV_XREG_WGS) {
       const int nrb = N / 16, per = (nrb + GEMV_XREG_WGS - 1) / GEMV_XREG_WGS;
       hipLaunchKernelGGL((gemv_xreg_kernel<GEMV_KS, GEMV_XS, GEMV_XREG_U, Epi, true>), dim3((nrb + per - 1) / per),
@@ -452,25 +468,13 @@ hipError_t launch_gemv(const f16* Wt, const f16* X, const NormIn* nin, const Att
     }
     return hipGetLastError();
   }
-  if (split) {
-    if (nin || ain) return hipErrorInvalidValue;
-    if (B >= GEMV_XREG_MINB && K <= 32 * GEMV_XS * GEMV_KS && N / 16 > GEMV_XREG_WGS) {
-      const int nrb = N / 16, per = (nrb + GEMV_XREG_WGS - 1) / GEMV_XREG_WGS;
-      hipLaunchKernelGGL((gemv_xreg_kernel<GEMV_KS, GEMV_XS, GEMV_XREG_U, Epi, false, true>),
-                         dim3((nrb + per - 1) / per), dim3(GEMV_KS * 64), 0, st, (const f16x8*)Wt, X, N, B, K, epi);
-      return hipGetLastError();
-    }
-    hipLaunchKernelGGL((gemv_kernel<GEMV_KS, GEMV_U, Epi, PRO_NONE, true>), dim3(N / 16),
-                       dim3(GEMV_KS * 64), 0, st, (const f16x8*)Wt, X, N, B, K, epi, NormIn{},
-                       AttnIn{});
-    return hipGetLastError();
-  }
   const dim3 grid(N / 16), block(GEMV_KS * 64);
   const size_t lds = (size_t)B * (K + 8) * 2;
   // Only the projections fed by a norm (QKV, W1|W3, logits) have a norm
   // prologue, and only Wo (residual epilogue) the attention combine.
-  constexpr bool kNorm = !std::is_same_v<Epi, EpiResidual> && !std::is_same_v<Epi, EpiStore>;
-  constexpr bool kAttn = std::is_same_v<Epi, EpiResidual>;
+  constexpr bool kAttn = std::is_same_v<Epi, EpiResidual>, kNorm = !kAttn;
+  // the fragment-order gate is written for 8 and more sequences only
+  constexpr bool kFewRows = !std::is_same_v<Epi, EpiSwiGLUFrag>;
   if (nin) {
     if constexpr (kNorm) {
       if (!gemv_norm_fits(B, K)) return hipErrorInvalidValue;
@@ -478,9 +482,9 @@ hipError_t launch_gemv(const f16* Wt, const f16* X, const NormIn* nin, const Att
         hipLaunchKernelGGL((gemv_kernel<GEMV_KS, GEMV_U, Epi, PRO_NORM + decltype(nb)::value, false>), grid, block,
                            lds, st, (const f16x8*)Wt, nullptr, N, B, K, epi, *nin, AttnIn{});
       };
-      if (B == 1) go(std::integral_constant<int, 1>{});
-      else if (B == 2) go(std::integral_constant<int, 2>{});
-      else go(std::integral_constant<int, GEMV_NORM_MAXB>{});
+      if (!kFewRows || B > 2) go(std::integral_constant<int, GEMV_NORM_MAXB>{});
+      else if (B == 1) go(std::integral_constant<int, kFewRows ? 1 : GEMV_NORM_MAXB>{});
+      else go(std::integral_constant<int, kFewRows ? 2 : GEMV_NORM_MAXB>{});
     } else {
       return hipErrorInvalidValue;
     }
@@ -515,40 +519,38 @@ bool gemv_attn_fits(int B, int K, int nch) {
 
 hipError_t gemv_residual(const f16* Wt, const f16* X, const AttnIn* ain, int N, int B, int K,
                          const EpiResidual& e, hipStream_t st, bool split, bool xfrag) {
-  return launch_gemv(Wt, X, nullptr, ain, N, B, K, e, st, split, xfrag);
+  if (split) return ain || xfrag ? hipErrorInvalidValue : launch_gemv_split(Wt, X, N, B, K, e, st);
+  return launch_gemv(Wt, X, nullptr, ain, N, B, K, e, st, xfrag);
 }
 hipError_t gemv_swiglu(const f16* Wt, const f16* X, const NormIn* nin, int N, int B, int K,
                        const EpiSwiGLU& e, hipStream_t st, bool split, bool xfrag) {
   if (e.frag) {
-    if (e.split || e.tap || B > 16 || e.hidden % 32) return hipErrorInvalidValue;
-    return launch_gemv(Wt, X, nin, nullptr, N, B, K, EpiSwiGLUFrag{e.gate}, st, split, xfrag);
+    if (split || e.split || e.tap || B < 8 || B > 16 || e.hidden % 32) return hipErrorInvalidValue;
+    return launch_gemv(Wt, X, nin, nullptr, N, B, K, EpiSwiGLUFrag{e.gate}, st, xfrag);
   }
-  return launch_gemv(Wt, X, nin, nullptr, N, B, K, e, st, split, xfrag);
+  if (split) return nin || xfrag ? hipErrorInvalidValue : launch_gemv_split(Wt, X, N, B, K, e, st);
+  return launch_gemv(Wt, X, nin, nullptr, N, B, K, e, st, xfrag);
 }
 hipError_t gemv_logits(const f16* Wt, const f16* X, const NormIn* nin, int N, int B, int K,
                        const EpiLogits& e, hipStream_t st, bool split, bool xfrag) {
-  return launch_gemv(Wt, X, nin, nullptr, N, B, K, e, st, split, xfrag);
+  if (split) return nin || xfrag ? hipErrorInvalidValue : launch_gemv_split(Wt, X, N, B, K, e, st);
+  return launch_gemv(Wt, X, nin, nullptr, N, B, K, e, st, xfrag);
 }
+// One position per sequence (d_pos), no fp32 tap; low parts of Q, K and V
+// exactly where X is split rows.
 hipError_t gemv_qkv(const f16* Wt, const f16* X, const NormIn* nin, int N, int B, int K,
                     const EpiQKV& e, hipStream_t st, bool split, bool xfrag) {
-  if (e.S < 1 || e.hd < 1) return hipErrorInvalidValue;
-  auto run = [&](auto dec, auto mode) {
-    EpiQKVAt<decltype(dec)::value, decltype(mode)::value> ep(e);
+  if (e.S < 1 || e.hd < 1 || !e.d_pos || e.mode() != (split ? EpiQKV::SPLIT : EpiQKV::PLAIN))
+    return hipErrorInvalidValue;
+  if (split) {
+    if (nin || xfrag) return hipErrorInvalidValue;
+    EpiQKVAt<true, EpiQKV::SPLIT> ep(e);
     ep.prepare();
-    return launch_gemv(Wt, X, nin, nullptr, N, B, K, ep, st, split, xfrag);
-  };
-  using Dec = std::integral_constant<bool, true>;
-  using Pre = std::integral_constant<bool, false>;
-  using Plain = std::integral_constant<int, EpiQKV::PLAIN>;
-  using Split = std::integral_constant<int, EpiQKV::SPLIT>;
-  using Full = std::integral_constant<int, EpiQKV::FULL>;
-  const int mode = e.mode();
-  if (e.d_pos)
-    return mode == EpiQKV::PLAIN ? run(Dec{}, Plain{}) : mode == EpiQKV::SPLIT ? run(Dec{}, Split{}) : run(Dec{}, Full{});
-  return mode == EpiQKV::PLAIN ? run(Pre{}, Plain{}) : mode == EpiQKV::SPLIT ? run(Pre{}, Split{}) : run(Pre{}, Full{});
-}
-hipError_t gemv_store(const f16* Wt, const f16* X, int N, int B, int K, float* C, hipStream_t st) {
-  return launch_gemv(Wt, X, nullptr, nullptr, N, B, K, EpiStore{C, N}, st);
+    return launch_gemv_split(Wt, X, N, B, K, ep, st);
+  }
+  EpiQKVAt<true, EpiQKV::PLAIN> ep(e);
+  ep.prepare();
+  return launch_gemv(Wt, X, nin, nullptr, N, B, K, ep, st, xfrag);
 }
 
 // ---- greedy token: reduce the argmax partials, advance the decode state ----

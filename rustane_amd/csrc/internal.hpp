@@ -105,7 +105,6 @@ hipError_t gemv_logits(const f16* Wt, const f16* X, const NormIn* nin, int N, in
 hipError_t gemv_qkv(const f16* Wt, const f16* X, const NormIn* nin, int N, int B, int K,
                     const EpiQKV& e, hipStream_t st, bool split = false,
                        bool xfrag = false);
-hipError_t gemv_store(const f16* Wt, const f16* X, int N, int B, int K, float* C, hipStream_t st);
 // Greedy token from the logits GEMV's argmax partials ([B][nblk] each). With
 // tok != NULL it also feeds the token back (tok, hist row pos - *d_pos0) and
 // advances *d_pos.

@@ -94,3 +94,28 @@ def test_inline_asm_leaves_m0_to_the_compiler():
                 copies += 1
                 assert '"{m0}"(' in stmt, (name, template)
     assert copies >= 2, "expected the direct-to-LDS copies in the sources"
+
+
+def test_decode_gemvs_are_built_for_the_rows_they_get():
+    """Split rows reach the projections of two-term layers and the logits, and
+    QKV with low parts gets no others; the fragment-order gate is never written
+    for one or two rows."""
+    names = [k["name"] for k in _kernel_metadata() if re.search(r"gemv(_xreg)?_kernel", k["name"])]
+    forms = {}
+    for n in names:
+        # <KS, U or XS, .., Epi, [PRO,] two flags>: the split flag is the last of
+        # the register-row kernel's and the first of the plain kernel's
+        m = re.search(r"gemv_(xreg_)?kernelI(?:Li\d+E)+NS_\d+(\w+?)(?:ILb(\d)ELi(\d)EE)?E(?:Li(\d+)E)?Lb(\d)ELb(\d)EE", n)
+        assert m, n
+        epi = m.group(2) + ("" if m.group(3) is None else f"<{m.group(3)},{m.group(4)}>")
+        split = (m.group(7) if m.group(1) else m.group(6)) == "1"
+        forms.setdefault(epi, set()).add((split, int(m.group(5) or 0)))
+    few, wide = {(False, 3), (False, 4)}, {(False, 0), (False, 10)}  # PRO_NORM + rows
+    assert forms == {
+        "EpiResidual": {(False, 0), (False, 1), (True, 0)},
+        "EpiSwiGLU": few | wide | {(True, 0)},
+        "EpiSwiGLUFrag": wide,
+        "EpiLogits": few | wide | {(True, 0)},
+        "EpiQKVAt<1,0>": few | wide,
+        "EpiQKVAt<1,1>": {(True, 0)},
+    }, forms
