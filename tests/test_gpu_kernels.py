@@ -261,9 +261,9 @@ def test_sdpa_op_on_staged_rope_tiles_spanning_sequences(gpu):
 
 @pytest.mark.parametrize("B,S", [(3, 700), (1, 512), (2, 100)])
 def test_sdpa_plain_stores_equal_tapped(gpu, B, S):
-    """The QKV GEMM's plain epilogue (no tap: Q, K and V^T addressed per
+    """The QKV GEMM's plain epilogue (no tap: Q, K and V rows addressed per
     token and per 32-feature block) and its tapped one (the fp32 tap too,
-    addressed per quad) must write the same fp16 Q, K and V^T: the attention
+    addressed per quad) must write the same fp16 Q, K and V: the attention
     output is compared bit for bit, on several tile shapes (256x256 staged
     tiles at 3 x 700 tokens, smaller ones below)."""
     import torch
@@ -311,6 +311,40 @@ def test_sdpa_ignores_stale_rows_past_the_sequence(gpu, S, hd, heads, kv):
         out = torch.empty((S, cfg.q_dim), dtype=torch.float16, device="cuda")
         hb.call("hb_op_sdpa_fwd", k.model.handle, 0, xn.data_ptr(), 1, S, out.data_ptr(), None)
         torch.cuda.synchronize()
+        outs.append(out.cpu().numpy())
+        k.model.close()
+        k.ctx.close()
+    assert np.isfinite(outs[0].astype(F32)).all()
+    np.testing.assert_array_equal(outs[0].view(np.uint16), outs[1].view(np.uint16))
+
+
+@pytest.mark.parametrize("hd,heads,kv", [(128, 8, 4), (64, 16, 16)])
+@pytest.mark.parametrize("S", [481, 500])
+def test_sdpa_ignores_stale_rows_on_full_grids(gpu, S, hd, heads, kv):
+    """The same on the instances that full grids take (ceil(blocks / 8) x heads
+    x sequences >= 256: whole key ranges per wave, three tile buffers): 16
+    blocks of 32, the last one with 1 or 20 rows of the sequence, behind a call
+    of 512 that leaves infinities and NaN in the rest of it."""
+    import torch
+    B = 256 // (2 * heads)
+    cfg = tiny_config(dim=512, hidden=256, heads=heads, kv_heads=kv, hd=hd, nlayers=1, seq=512, vocab=256)
+    w = ModelWeights.synthetic(cfg, seed=80, std=0.02)
+    xn = to_dev(f16_round(np.random.default_rng(14).standard_normal((B * S, cfg.dim))), torch.float16)
+    bad = torch.full((B * cfg.seq, cfg.dim), float("inf"), dtype=torch.float16, device="cuda")
+    print(f"sdpa stale rows: B={B} S={S} hd={hd} heads={heads}/{kv}", flush=True)
+    outs = []
+    for spoil in (False, True):
+        k = CompiledKernels.compile(cfg)
+        k.ctx.set_stream(gpu.stream())
+        k.ensure_weights(w)
+        if spoil:
+            scrap = torch.empty((B * cfg.seq, cfg.q_dim), dtype=torch.float16, device="cuda")
+            hb.call("hb_op_sdpa_fwd", k.model.handle, 0, bad.data_ptr(), B, cfg.seq, scrap.data_ptr(), None)
+        out = torch.empty((B * S, cfg.q_dim), dtype=torch.float16, device="cuda")
+        hb.call("hb_op_sdpa_fwd", k.model.handle, 0, xn.data_ptr(), B, S, out.data_ptr(), None)
+        torch.cuda.synchronize()
+        if spoil:
+            assert not torch.isfinite(scrap).all()  # the longer call did leave them
         outs.append(out.cpu().numpy())
         k.model.close()
         k.ctx.close()

@@ -327,6 +327,37 @@ def test_decode_results_reach_any_buffer(m48, B):
             np.testing.assert_array_equal(ids, exp_ids)
 
 
+@pytest.mark.parametrize("hd,heads,kv", [(128, 8, 2), (64, 16, 16)])
+@pytest.mark.parametrize("B,S", [(1, 33), (16, 33), (8, 481), (16, 481)])
+def test_prefill_ignores_stale_cache_rows(gpu, B, S, hd, heads, kv):
+    """A cache that a longer prompt filled with NaN, then reset: a shorter
+    prompt of a ragged length and two steps behind it equal a fresh cache's bit
+    for bit, in the two-term first layer (low parts stale too) and the plain
+    second, on small grids and on full ones (16 x 481 with 8 heads, 8 and 16 x
+    481 with 16: 256 and more groups of 8 query blocks)."""
+    cfg = tiny_config(dim=256, hidden=256, heads=heads, kv_heads=kv, hd=hd, nlayers=2, seq=512, vocab=256)
+    w = ModelWeights.synthetic(cfg, seed=81, std=0.02)
+    BAD = 7  # a token whose embedding row makes its normalised row NaN
+    w.embed.reshape(cfg.vocab, cfg.dim)[BAD] = np.inf
+    tok = tokens_for(cfg, B * (S + 2), seed=29).reshape(B, S + 2)
+    tok[tok == BAD] = BAD + 1
+    keep = np.arange(cfg.vocab) != BAD  # the tied head's column BAD is not finite in either
+    print(f"prefill stale rows: B={B} S={S} hd={hd} heads={heads}/{kv}", flush=True)
+    outs = []
+    for spoil in (False, True):
+        k = CompiledKernels.compile(cfg)
+        k.ensure_weights(w)
+        dec = E.Decoder(k, batch=B, ctx_max=cfg.seq)
+        if spoil:
+            bad = dec.prefill(np.full((B, cfg.seq), BAD, np.uint32))[0]
+            assert np.isnan(bad[:, keep]).all()
+            dec.kv.reset()
+        got = [dec.prefill(tok[:, :S])[0]] + [dec.step(np.ascontiguousarray(tok[:, S + i]))[0] for i in (0, 1)]
+        outs.append(np.stack(got)[..., keep])
+    assert np.isfinite(outs[0]).all()
+    np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
 @pytest.mark.parametrize("kind", ["device", "pinned"])
 def test_decode_results_reach_device_and_pinned_buffers(m48, kind):
     """Each of the two results may go to device memory (the runtime copies it)

@@ -71,6 +71,23 @@ def test_gemm_kernels_keep_accumulators_in_registers():
         assert int(k["private_segment_fixed_size"]) <= 128, (k["name"], k["private_segment_fixed_size"])
 
 
+def test_register_array_kernels_use_no_scratch():
+    """These keep tiles, rows or accumulators in registers up to the limit of
+    their occupancy: nothing may be spilled, and an instance meant to run two
+    workgroups of 4 waves to a CU needs at most 256 registers a lane."""
+    ks = _kernel_metadata()
+    for name, least in (("attn_prefill_kernel", 8), ("attn_bwd_dq_kernel", 4), ("attn_bwd_dkv_kernel", 4),
+                        ("attn_decode_kernel", 8), ("ce_backward_kernel", 3), ("gemv_xreg_kernel", 11)):
+        mine = [k for k in ks if name in k["name"]]
+        assert len(mine) >= least, (name, len(mine))
+        for k in mine:
+            assert int(k["private_segment_fixed_size"]) == 0, (k["name"], k["private_segment_fixed_size"])
+            two = ("attn_bwd_dq" in name or ("attn_bwd_dkv" in name and "Li4ELi1E" in k["name"]) or
+                   ("attn_prefill" in name and "ELb0ELi" in k["name"]))
+            if two:
+                assert int(k["vgpr_count"]) <= 256, (k["name"], k["vgpr_count"])
+
+
 def test_kernels_fit_the_cu():
     for k in _kernel_metadata():
         assert int(k["group_segment_fixed_size"]) <= 160 * 1024, k["name"]
