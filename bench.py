@@ -351,11 +351,14 @@ def time_dominant_kernel(k, cfg, T, launches, stream):
     achieved = up_flops / (up_ms / 1e3) / 1e12
     log(f"[bench] ffn-up GEMM {T}x{2*cfg.hidden}x{cfg.dim}: {up_ms*1e3:.1f} us/launch, "
         f"{achieved:.1f} TFLOP/s ({achieved/2500*100:.1f}% of dense fp16 peak)")
+    counted = (cfg.dim, cfg.hidden, T) == (4096, 11008, 512)  # the launch the counters were read on
     roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": 2500.0, "unit": "TFLOP/s",
-                "frac": round(achieved / 2500.0, 4), "traffic": DOMINANT_TRAFFIC_BYTES,
+                "frac": round(achieved / 2500.0, 4), "traffic": DOMINANT_TRAFFIC_BYTES if counted else None,
                 "traffic_source": "rocprofv3 FETCH_SIZE + WRITE_SIZE of this kernel, scaled by a 1 GiB copy "
-                                  "(profiles/ffn_up_gemm_7b_b1_counters.md), not measured in this run",
-                "kernel": "gemm_nt_kernel<192,256,2,2,EpiSwiGLU> (FFN up, W1|W3 + SwiGLU)",
+                                  "(profiles/ffn_up_gemm_7b_b1_counters.md), not measured in this run"
+                                  if counted else None,
+                "kernel": ("gemm_nt_kernel<192,256,EpiSwiGLU>" if counted else "prefill GEMM, EpiSwiGLU")
+                          + " (FFN up, W1|W3 + SwiGLU)",
                 "flop_per_launch": up_flops, "us_per_launch": round(up_ms * 1e3, 2),
                 "timing": "us_per_launch: launches back to back (HIP events around a graph of them); "
                           "us_per_launch_in_forward: inside the forward, from hb_forward_timed"}

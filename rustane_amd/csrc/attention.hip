@@ -30,7 +30,8 @@ namespace hb {
 // sustains — while splitting the key range over PK waves keeps the chain of
 // dependent key blocks at half the row; the key halves merge through LDS at
 // the end (the same rescaling an online softmax applies between blocks).
-// Fragments are read from XOR-swizzled LDS without bank conflicts. Workgroups
+// K fragments are read from XOR-swizzled LDS without bank conflicts, the
+// transposed V reads take 6 conflict cycles each. Workgroups
 // of 4 waves leave room for two or three on a CU, whose MFMAs and softmaxes
 // overlap.
 //

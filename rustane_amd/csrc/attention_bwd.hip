@@ -16,9 +16,11 @@
 // (TrFrag), so no transposed copies exist in memory or LDS.
 //
 // Tiles go from global memory straight into LDS (dma_1k) one or two
-// iterations ahead, with one barrier per iteration; a workgroup is 4 waves of
-// at most 256 registers, two workgroups to a CU, so that one's softmax and
-// waits run under the other's MFMAs. The predecessors (register-staged
+// iterations ahead, with one barrier per iteration; a workgroup is 4 waves. The
+// dQ instances and the wide dK/dV ones (PH = 1) use at most 256 registers, two
+// workgroups to a CU, so that one's softmax and waits run under the other's
+// MFMAs; dK/dV with two query halves takes 384 at hd = 128, one to a CU, on
+// grids that give a CU no second one. The predecessors (register-staged
 // double-buffered tiles, transposed copies, one workgroup of 4 waves per CU)
 // spent most of an iteration waiting: 20 heads x 2048 of 128, us: dQ 344 ->
 // 154, dK/dV 336 -> 121; 32 heads x 4 x 512, 70 -> 64 and 99 -> 51.
@@ -86,8 +88,8 @@ __global__ __launch_bounds__(PQ * PK * 64, 2) void attn_bwd_dq_kernel(AttnBwd p)
   const int qs = wave % PQ, kh = wave / PQ;
   const int nqb = (p.S + 31) / 32, ngr = (nqb + PQ - 1) / PQ;
   const int gr = ngr - 1 - blockIdx.x;  // heaviest groups first
-  // query blocks gr, gr + ngr, ... (as in the forward kernel: groups of
-  // nearly equal causal work)
+  // query blocks gr, gr + ngr, ...: every group spans the sequence, so the
+  // groups' causal work is nearly equal
   const int qb = gr + ngr * qs;
   const bool active = qb < nqb;
   const int nkb = gr + ngr * min(PQ - 1, (nqb - 1 - gr) / ngr) + 1;

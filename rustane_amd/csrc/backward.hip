@@ -113,7 +113,10 @@ hipError_t cast_transpose(const float* src, int R, int C, float scale, f16* rm, 
 // HBM-bound: 4 V bytes read and 2 Vp written per position. The row stays in
 // registers (NV float4 per thread, V <= 2048 * NV), so it is read once with
 // 16-byte loads and each exponential is taken once: 2048 x 32000 from 230 us
-// (three passes of 4-byte loads) to 106. NV = 0: any V, in three passes.
+// (three passes of 4-byte loads by 256 threads) to 106. NV = 0: any V, in three
+// passes. 1024 positions, us, the 256-thread passes -> now: V = 8256 36 -> 19,
+// 16384 71 -> 31, 32000 139 -> 53 in registers; 33024 143 -> 84, 50304 231 ->
+// 139, 128256 830 -> 513 in passes.
 constexpr int CE_NT = 512;
 template <int NV>
 __global__ __launch_bounds__(CE_NT) void ce_backward_kernel(const float* __restrict__ logits,

@@ -153,10 +153,13 @@ int gemm_splits(int N, int T, int K) {
 }
 
 // The residual + RMSNorm projections (gemm_residual_norm): a long reduction
-// (K >= 2N) whose 128x256 tiles in S splits fill the CUs exactly takes those
-// (7B W2 at 512 tokens: 64 tiles x 4 splits instead of 128 of 128x128 x 2;
-// GEMM alone 54 -> 45.5 us: the wider tile's main loop outweighs the reduce
-// reading 4 partials instead of 2; Wo, K = N, gains less).
+// (K >= 2N) takes the split count in which blocks of 256 features x 128 tokens
+// fill the CUs exactly (7B W2 at 512 tokens: 64 blocks, 4 splits instead of 2;
+// GEMM alone 54 -> 45.5 us, run on 64 tiles of 128x256 as gemm_tile picks them:
+// the wider tile's main loop outweighs the reduce reading 4 partials instead of
+// 2; Wo, K = N, gains less). The block shape is that of the tile these launches
+// first ran on and is kept because the count fixes the order of the forward's
+// sums; where it does not divide the CUs, gemm_splits' count stands.
 int gemm_norm_splits(int N, int T, int K) {
   const int S = gemm_splits(N, T, K);
   if (S <= 1 || K < 2 * N) return S;

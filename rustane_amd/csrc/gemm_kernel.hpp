@@ -19,8 +19,10 @@
 // halves of each row meet the same weights. kw = K otherwise.
 //
 // LDS rows are 128 B (64 halfs) of eight 16-byte chunks; chunk c of row r is
-// stored at c ^ swz(r), which keeps both the loaders' ds_write_b128 and the
-// MFMA operands' ds_read_b128 free of bank conflicts for 32- and 64-bank LDS.
+// stored at c ^ swz(r), which keeps the ds_write_b128 of gemm_nt_kernel_reg and
+// its 32-row operands' ds_read_b128 free of bank conflicts; the 16-row operand
+// reads of gemm_nt_kernel take 4 conflict cycles each (SQ_LDS_BANK_CONFLICT is
+// 4.00 x SQ_INSTS_LDS in every tile).
 #pragma once
 #include <type_traits>
 
@@ -161,16 +163,21 @@ struct GemmPlan {
 // have read it, about 1.5 slices before its next use, and the waits count
 // copies (dma_wait) instead of draining them.
 //
-// What bounds it: the chip's power limit. MFMA busy is ~83% of the active
-// cycles (63% in the 4-wave register-staged kernel below at 4096 tokens), and
-// the clock then settles with the energy per flop, so the instruction shape
-// matters: 16x16x32 touches half the accumulator registers per flop of
-// 32x32x16 and took the same schedule from 393 to 328 us on 12288 x 4096 x
-// 4096 (results bit-identical), and consecutive MFMAs that keep the token
-// operand another 2-4%. Before -> after, fp32 output, back to back on one
-// box (N x T x K): 12288 x 4096 x 4096 413 -> 307 us (998 -> 1344 TFLOP/s),
-// 22016 x 4096 x 4096 691 -> 608 us, 4096 x 4096 x 11008 287 -> 256 us,
-// 8192^3 886 -> 751 us (1463 TFLOP/s), 22016 x 512 x 4096 87 -> 76 us.
+// What bounds it: the matrix cores under the chip's power limit. MFMA busy is
+// 64-70% of the active cycles at 4096 tokens and 53% at 512 (60-70% and 50% in
+// the 4-wave register-staged kernel on these shapes), in 6% fewer cycles; the
+// rest of the gain is the clock, which settles with the energy per flop,
+// so the instruction shape matters: 16x16x32 touches half the accumulator
+// registers per flop of 32x32x16 and took the same schedule from 393 to 328 us
+// on 12288 x 4096 x 4096 (results bit-identical), and consecutive MFMAs that
+// keep the token operand another 2-4%. The clock follows the operand values
+// too: all-zero operands run 16-30% faster. Register-staged kernel -> this one,
+// fp32 output, back to back on one box, weights and activations N(0, 1) (N x T x
+// K): 12288 x 4096 x 4096 357 -> 323 us (1278 TFLOP/s), 22016 x 4096 x 4096 683
+// -> 617, 4096 x 4096 x 11008 299 -> 264, 8192^3 885 -> 793 (1387 TFLOP/s),
+// 22016 x 512 x 4096 90 -> 79; 12288 x 512 x 4096, one round of 192x128 tiles,
+// 57 -> 58. Weights N(0, 0.02): 353 -> 313, 683 -> 623, 302 -> 264, 893 -> 800,
+// 89 -> 79 and 55 -> 55.
 //
 // LDS is written by copies the compiler does not see: its address enters
 // their asm, and every copy is waited for before the barrier that precedes its
