@@ -22,8 +22,9 @@
 // MFMAs; dK/dV with two query halves takes 384 at hd = 128, one to a CU, on
 // grids that give a CU no second one. The predecessors (register-staged
 // double-buffered tiles, transposed copies, one workgroup of 4 waves per CU)
-// spent most of an iteration waiting: 20 heads x 2048 of 128, us: dQ 344 ->
-// 154, dK/dV 336 -> 121; 32 heads x 4 x 512, 70 -> 64 and 99 -> 51.
+// spent most of an iteration waiting: 20 heads x 2048 of 128, us: dQ 337 ->
+// 139, dK/dV 326 -> 118; 32 heads x 4 x 512, 70 -> 58 and 98 -> 49; 32 heads x
+// 512, split ranges, 45 -> 34 and 42 -> 31.
 //
 // attn_bwd_dq_kernel, per (PQ query blocks, head, sequence), PQ x PK waves
 // (PK key parts): S^T = K Q^T and dP^T = V dO^T per key block, two passes
