@@ -61,6 +61,7 @@ struct GemmTile {
   float slice_us, tile_us;
 };
 extern const GemmTile GEMM_TILES[6];
+constexpr int GEMM_192x256 = 1, GEMM_128x256 = 2;  // indices into it
 // The fastest tile of a product in `splits` K splits, and its predicted time.
 GemmChoice gemm_tile(int N, int T, int K, int splits, float* us = nullptr);
 

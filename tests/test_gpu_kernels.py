@@ -352,6 +352,38 @@ def test_sdpa_ignores_stale_rows_on_full_grids(gpu, S, hd, heads, kv):
     np.testing.assert_array_equal(outs[0].view(np.uint16), outs[1].view(np.uint16))
 
 
+@pytest.mark.parametrize("T", [128, 129, 200, 256, 257])
+def test_head_logits_exact_around_one_token_tile(gpu, T):
+    """Logits of 129 to 256 tokens run on 192x256 tiles (167 of them at 32000
+    columns, the last one ragged), the counts beside them on other tiles. Small
+    integers: exact in fp32 in any order of the sums."""
+    import torch
+    cfg = tiny_config(dim=128, hidden=256, heads=2, nlayers=1, seq=64, vocab=32000)
+    k = CompiledKernels.compile(cfg)
+    k.ctx.set_stream(gpu.stream())
+    w = ModelWeights.synthetic(cfg, seed=83, std=0.02)
+    rng = np.random.default_rng(T)
+    w.embed[:] = rng.integers(-3, 4, w.embed.size)
+    k.ensure_weights(w)
+    xn = rng.integers(-3, 4, (T, cfg.dim)).astype(F32)
+    tgt = rng.integers(0, cfg.vocab, T).astype(np.int32)
+    print(f"head tiles T={T}", flush=True)
+    dxn, dtgt = to_dev(xn, torch.float16), to_dev(tgt)
+    logits = torch.full((T, cfg.vocab), float("nan"), device="cuda")
+    losses = torch.empty(T, device="cuda")
+    hb.call("hb_op_logits_ce", k.model.handle, dxn.data_ptr(), dtgt.data_ptr(), T, logits.data_ptr(), losses.data_ptr())
+    torch.cuda.synchronize()
+    ref = xn @ w.embed.reshape(cfg.vocab, cfg.dim).T
+    np.testing.assert_array_equal(logits.cpu().numpy(), ref)
+    r = ref.astype(np.float64)
+    want = np.log(np.exp(r - r.max(1, keepdims=True)).sum(1)) + r.max(1) - r[np.arange(T), tgt]
+    # 32000 fp32 terms behind one rescale per batch: a few ulp of the sum, and an
+    # ulp of the loss (up to ~300)
+    np.testing.assert_allclose(losses.cpu().numpy(), want, rtol=1e-6, atol=1e-5)
+    k.model.close()
+    k.ctx.close()
+
+
 def test_logits_ce_op_matches_oracle(tiny):
     import torch
     cfg, k, w = tiny
