@@ -113,15 +113,23 @@ __global__ __launch_bounds__(256) void splitk_reduce_norm_kernel(const float* __
 // 42. 192x128 and 128x128 workgroups run two to a CU, one's epilogue under the
 // other's main loop (tile_us): QKV of 600M at 4096 tokens 88 us on 192x128
 // with its attention, 94 on 192x256.
-const GemmTile GEMM_TILES[6] = {{256, 256, 1.43f, 12.f}, {192, 256, 1.11f, 10.f},  {128, 256, 0.83f, 8.f},
-                                {192, 128, 0.64f, 5.5f}, {128, 128, 0.49f, 5.f},   {64, 128, 0.42f, 4.5f}};
+// Unsplit products have a seventh tile, 256x128 (launch_gemm): 513 to 640 tokens
+// are five columns of it, where 256-token tiles run 17-33% padding and smaller
+// ones a second round. Blocks of the other tiles -> 256x128, us, one stream: 7B
+// attention block at 513 / 640 tokens 86.4 / 94.9 -> 79.2 / 84.8, GQA FFN 63.5 /
+// 70.7 -> 61.2 / 66.1, 7B FFN 225.9 / 242.7 -> 225.6 / 238.4. Forced on the QKV and
+// W1|W3 products at 45 to 2048 other tokens it is level or up to 70% slower: its
+// constants are fitted at K = 2048 and 4096, and its tile_us keeps it from shorter K.
+const GemmTile GEMM_TILES[GEMM_NTILES] = {{256, 256, 1.43f, 12.f}, {192, 256, 1.11f, 10.f}, {128, 256, 0.83f, 8.f},
+                                          {192, 128, 0.64f, 5.5f}, {128, 128, 0.49f, 5.f},  {64, 128, 0.42f, 4.5f},
+                                          {256, 128, 0.81f, 15.f}};
 static constexpr int GEMM_CUS = 256;  // MI355X compute units
 
-GemmChoice gemm_tile(int N, int T, int K, int S, float* us) {
+GemmChoice gemm_tile(int N, int T, int K, int S, float* us, int tiles) {
   const int kq = (K / 64 + S - 1) / S;
   GemmChoice best{0, S};
   float best_us = INFINITY;
-  for (int i = 0; i < 6; ++i) {
+  for (int i = 0; i < tiles; ++i) {
     const GemmTile& g = GEMM_TILES[i];
     const long n = ntiles(N, T, g.ft, g.tt) * S;
     const float fill = (float)(n % GEMM_CUS) / GEMM_CUS;

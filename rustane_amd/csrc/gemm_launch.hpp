@@ -9,7 +9,7 @@ namespace hb {
 
 // The tiles gemm_nt_kernel runs; the others run on gemm_nt_kernel_reg.
 template <int FT, int TT>
-constexpr bool kDmaTile = (TT == 256 && FT >= 128) || (FT == 192 && TT == 128);
+constexpr bool kDmaTile = (TT == 256 && FT >= 128) || (TT == 128 && FT >= 192);
 
 // kw: W's row length; K (the X row length and the reduction length) is kw,
 // or 2 * kw for split X rows (gemm_kernel.hpp). 0 means K.
@@ -60,10 +60,11 @@ struct GemmTile {
   int ft, tt;
   float slice_us, tile_us;
 };
-extern const GemmTile GEMM_TILES[6];
-constexpr int GEMM_192x256 = 1, GEMM_128x256 = 2;  // indices into it
-// The fastest tile of a product in `splits` K splits, and its predicted time.
-GemmChoice gemm_tile(int N, int T, int K, int splits, float* us = nullptr);
+constexpr int GEMM_NTILES = 7, GEMM_192x256 = 1, GEMM_128x256 = 2, GEMM_256x128 = 6;  // 6: launch_gemm's only
+extern const GemmTile GEMM_TILES[GEMM_NTILES];
+// The fastest of the first `tiles` tiles of a product in `splits` K splits, and its
+// predicted time.
+GemmChoice gemm_tile(int N, int T, int K, int splits, float* us = nullptr, int tiles = GEMM_256x128);
 
 template <class Epi>
 static hipError_t launch_choice(GemmChoice c, const f16* W, const f16* X, int N, int T, int K, const Epi& epi,
@@ -86,8 +87,13 @@ template <class Epi>
 static hipError_t launch_gemm(const f16* W, const f16* X, int N, int T, int K, const Epi& epi,
                               hipStream_t st, int kw = 0, int* tiles = nullptr) {
   if (!gemm_fits(N, T, K)) return hipErrorInvalidValue;
-  const GemmChoice c = gemm_tile(N, T, K, 1);
+  // 256x128 fills one round of the CUs where no other tile does; not where the
+  // tile sets the order of a sum of squares
+  constexpr bool tall = !EpiSumSq<Epi>::value;
+  const GemmChoice c = gemm_tile(N, T, K, 1, nullptr, tall ? GEMM_NTILES : GEMM_256x128);
   if (tiles) *tiles = (int)ntiles(N, T, GEMM_TILES[c.tile].ft, GEMM_TILES[c.tile].tt);
+  if constexpr (tall)
+    if (c.tile == GEMM_256x128) return launch_tile<256, 128>(W, X, N, T, K, epi, st, 1, kw);
   return launch_choice(c, W, X, N, T, K, epi, st, kw);
 }
 

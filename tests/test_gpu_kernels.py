@@ -72,6 +72,24 @@ def test_gemm_nt_tiles_exact(gpu, M, N, K):
     np.testing.assert_array_equal(dc.cpu().numpy(), a @ b.T)
 
 
+@pytest.mark.parametrize("K", [1920, 1984])  # 30 and 31 slices: even and odd ends of the two-slice loop
+@pytest.mark.parametrize("M", [513, 600, 639])
+def test_gemm_nt_one_round_of_256x128_tiles_exact(gpu, M, K):
+    """N = 12284 at 513 to 640 tokens: 48 x 5 tiles of 256x128, the last row and
+    the last column of them ragged. Exact as above."""
+    import torch
+    print(f"gemm 256x128 tiles M={M} K={K}", flush=True)
+    rng = np.random.default_rng(M + K)
+    N = 12284
+    a = rng.integers(-3, 4, (M, K)).astype(np.float32)
+    b = rng.integers(-3, 4, (N, K)).astype(np.float32)
+    da, db = to_dev(a, torch.float16), to_dev(b, torch.float16)
+    dc = torch.full((M, N), float("nan"), device="cuda")
+    hb.call("hb_op_gemm_nt", gpu.handle, da.data_ptr(), db.data_ptr(), dc.data_ptr(), M, N, K)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(dc.cpu().numpy(), a @ b.T)
+
+
 def test_gemm_nt_mfma_layout_one_hot(gpu):
     """A one-hot A row selects exactly one B row: catches any lane/register
     layout mistake in the MFMA fragments independently of rounding."""
@@ -251,6 +269,42 @@ def test_sdpa_op_on_staged_rope_tiles_spanning_sequences(gpu):
         s = O.sdpa_fwd(oc, xn[rows].T, f16_round(lw.wq), f16_round(lw.wk), f16_round(lw.wv), S)
         print(f"sequence {b}: max|dq| {np.abs(t[rows, :q] - s['q_rope'].T).max():.2e} "
               f"max|dattn| {np.abs(attn[rows] - s['attn'].T).max():.2e}", flush=True)
+        np.testing.assert_allclose(t[rows, :q], s["q_rope"].T, atol=2e-3)
+        np.testing.assert_allclose(t[rows, q:q + kv], s["k_rope"].T, atol=2e-3)
+        np.testing.assert_allclose(t[rows, q + kv:], s["v"].T, atol=2e-3)
+        np.testing.assert_allclose(attn[rows], s["attn"].T, atol=3e-3)
+    k.model.close()
+    k.ctx.close()
+
+
+def test_sdpa_op_on_256x128_rope_tiles_spanning_sequences(gpu):
+    """The same on 32 heads at 3 x 200 tokens (N = 12288, K = 2048: 240 tiles of
+    256x128, whose table slices are staged too), with a 128-token tile holding
+    the end of one sequence and the start of the next."""
+    import torch
+    cfg = tiny_config(dim=2048, hidden=256, heads=32, hd=128, nlayers=1, seq=200, vocab=256)
+    k = CompiledKernels.compile(cfg)
+    k.ctx.set_stream(gpu.stream())
+    w = ModelWeights.synthetic(cfg, seed=84, std=0.02)
+    k.ensure_weights(w)
+    oc = oracle_cfg(cfg)
+    lw = oracle_weights(w).layers[0]
+    B, S = 3, cfg.seq
+    xn = f16_round(np.random.default_rng(14).standard_normal((B * S, cfg.dim)) * 0.5)
+    dxn = to_dev(xn, torch.float16)
+    dattn = torch.empty((B * S, cfg.q_dim), dtype=torch.float16, device="cuda")
+    tap = torch.empty((B * S, cfg.q_dim + 2 * cfg.kv_dim), device="cuda")
+    print("sdpa on 256x128 tiles", flush=True)
+    hb.call("hb_op_sdpa_fwd", k.model.handle, 0, dxn.data_ptr(), B, S, dattn.data_ptr(), tap.data_ptr())
+    torch.cuda.synchronize()
+    t, attn = tap.cpu().numpy(), dattn.float().cpu().numpy()
+    hb.call("hb_op_sdpa_fwd", k.model.handle, 0, dxn.data_ptr(), B, S, dattn.data_ptr(), None)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(dattn.float().cpu().numpy(), attn)  # the plain epilogue stores the same
+    q, kv = cfg.q_dim, cfg.kv_dim
+    for b in range(B):
+        rows = slice(b * S, (b + 1) * S)
+        s = O.sdpa_fwd(oc, xn[rows].T, f16_round(lw.wq), f16_round(lw.wk), f16_round(lw.wv), S)
         np.testing.assert_allclose(t[rows, :q], s["q_rope"].T, atol=2e-3)
         np.testing.assert_allclose(t[rows, q:q + kv], s["k_rope"].T, atol=2e-3)
         np.testing.assert_allclose(t[rows, q + kv:], s["v"].T, atol=2e-3)
